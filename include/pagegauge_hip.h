@@ -221,6 +221,19 @@ int32_t pg_token_major_centers_noalloc(const void* key, int64_t key_token_stride
                                        int64_t tokens, int32_t heads, void* key_center,
                                        void* value_center, void* stream);
 
+/* Causal self-attention of one prompt (the prompt pass that fills the caches;
+ * plain torch operators in the reference's TransformerDecoder,
+ * scripts/benchmark_page_gauge_transformer.py).  query / out: [tokens,
+ * query_heads, 128] fp16, key / value: [tokens, kv_heads, 128] fp16, dense
+ * heads, token rows *_stride elements apart (multiples of 8; rows 16-byte
+ * aligned; a K or V slice of a fused QKV projection will do).  Query head h
+ * reads KV head h / 4 (GQA group 4 only).  Scores, softmax and output sums
+ * are float32; probabilities enter the value product as FP16. */
+int32_t pg_causal_attention(const void* query, int64_t query_stride, const void* key,
+                            int64_t key_stride, const void* value, int64_t value_stride,
+                            void* out, int64_t out_stride, int32_t tokens, int32_t query_heads,
+                            int32_t kv_heads, float sm_scale, void* stream);
+
 /* ------------------------------------------------------------------------
  * Paged decode (K1) and the split scheduler (S).
  * ---------------------------------------------------------------------- */

@@ -66,6 +66,7 @@ SOURCES = {
     # variant against it), same output bits
     "pg_decode.hip": ["-mllvm", "-amdgpu-sched-strategy=max-memory-clause"],
     "pg_decoder.hip": [],
+    "pg_prefill.hip": [],
 }
 
 BENCH_SOURCES = {

@@ -1,0 +1,328 @@
+// Prompt (prefill) attention for gfx950: causal attention of a whole prompt,
+// [T, Hq, 128] x [T, Hkv, 128] FP16 with GQA group 4 and a float32 online
+// softmax (the prompt pass of scripts/benchmark_page_gauge_transformer.py's
+// TransformerDecoder).
+#include "pg_common.h"
+
+namespace pg {
+namespace {
+
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef short v4s __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+
+#define PG_LDS __attribute__((address_space(3)))
+#define PG_GLOBAL __attribute__((address_space(1)))
+
+constexpr int kTileKeys = 64;
+constexpr int kTileBytes = kTileKeys * kHeadDim * 2;     // 16 KiB
+constexpr float kRescaleLimit = 8.0f;                    // log2
+constexpr float kNegInf = -__builtin_huge_valf();
+
+struct AttentionArgs {
+  const uint16_t* query;
+  const uint16_t* key;
+  const uint16_t* value;
+  uint16_t* out;
+  int64_t query_stride;
+  int64_t key_stride;
+  int64_t value_stride;
+  int64_t out_stride;
+  int tokens;
+  int kv_heads;
+  int blocks;          // query blocks
+  float scale_log2;
+};
+
+// One workgroup per (KV head, block of queries): its waves are the 4 query
+// heads of the group times blocks of 32 queries, and they share every K and V
+// tile of 64 keys through LDS.  A wave keeps its queries as the B operand of
+// v_mfma_f32_32x32x16_f16 and computes S^T = K Q^T, so that a lane holds 32
+// scores of ONE query: the softmax reduces in registers plus one swap with
+// the lane 32 away, the running maximum and the rescale are per-lane scalars,
+// and the probabilities are, register for register, the B operand of
+// O^T += V^T P^T (V^T through transposing LDS reads, keys permuted alike).
+//
+// K and V tiles go from memory to LDS directly, double-buffered, one barrier
+// per tile; the 16-byte chunks of a row are swizzled by the row (in the
+// source address) so that neither the K reads (8 rows per access) nor the
+// transposing V reads (4 rows x 32 bytes) meet in a bank.  The scores of tile
+// j + 1 are computed beside the softmax of tile j: the two halves of the work
+// use the matrix cores and the VALU (exp2 at a quarter rate) for about the
+// same time, which is what bounds the kernel, with the LDS reads (32 KiB per
+// wave and tile) close behind.
+//
+// The running maximum is raised only when a score exceeds it by more than
+// 2^8 (probabilities then reach 256, which FP16 holds at the same relative
+// precision): most tiles skip the rescale of the accumulators.
+//
+// Blocks are dispatched longest first, and KV heads vary fastest, so that with
+// 8 heads each XCD works on one head's keys and values.
+//
+// Measured, 32 query and 8 KV heads: 16384 tokens 1.99 ms (1105 TFLOP/s of the
+// causal half; about 38 ms as matmul, mask, softmax and matmul launches over
+// float32 scores in memory), 4096 tokens 139 us (985), 1000 tokens 23 us
+// (340, too few workgroups).
+template <int kWaves>
+__global__ __launch_bounds__(kWave * kWaves, 2) void causal_attention_kernel(AttentionArgs a) {
+  constexpr int kQueries = 32 * (kWaves / kGqa);   // query rows per workgroup
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[4 * kTileBytes];   // K0 K1 V0 V1
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int lane = threadIdx.x % kWave;
+  const int kv = blockIdx.x % a.kv_heads;
+  const int block = a.blocks - 1 - blockIdx.x / a.kv_heads;
+  const int head = kv * kGqa + wave % kGqa;
+  const int q0 = block * kQueries + 32 * (wave / kGqa);
+  const int half = lane >> 5;
+  const int column = lane & 31;
+  const int q = q0 + column;
+  const int last = a.tokens - 1;
+  // key tiles that any row of the workgroup sees
+  const int tiles = (min((block + 1) * kQueries, a.tokens) + kTileKeys - 1) / kTileKeys;
+
+  v8h qf[8];
+  const uint16_t* qp = a.query + static_cast<int64_t>(min(q, last)) * a.query_stride + head * kHeadDim + 8 * half;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) qf[k] = *reinterpret_cast<const v8h*>(qp + 16 * k);
+
+  // direct-to-LDS tile loads: one instruction fills 4 rows
+  const uint16_t* kg = a.key + kv * kHeadDim;
+  const uint16_t* vg = a.value + kv * kHeadDim;
+  const int lrow = lane >> 4;
+  const int lchunk = lane & 15;
+  constexpr int kLoads = 16 / kWaves;      // per wave and tensor
+  auto load_k = [&](int tile, int buffer) {
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const int row = 4 * (wave * kLoads + i) + lrow;
+      const int key = min(tile * kTileKeys + row, last);
+      const uint16_t* src = kg + static_cast<int64_t>(key) * a.key_stride + 8 * (lchunk ^ (row & 15));
+      __builtin_amdgcn_global_load_lds(
+          (const PG_GLOBAL void*)src,
+          (PG_LDS void*)(lds + buffer * kTileBytes + 1024 * (wave * kLoads + i)), 16, 0, 0);
+    }
+  };
+  auto load_v = [&](int tile, int buffer) {
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const int row = 4 * (wave * kLoads + i) + lrow;
+      const int key = min(tile * kTileKeys + row, last);
+      const uint16_t* src = vg + static_cast<int64_t>(key) * a.value_stride + 8 * (lchunk ^ (4 * (row & 3)));
+      __builtin_amdgcn_global_load_lds(
+          (const PG_GLOBAL void*)src,
+          (PG_LDS void*)(lds + (2 + buffer) * kTileBytes + 1024 * (wave * kLoads + i)), 16, 0, 0);
+    }
+  };
+  // LDS read offsets
+  uint32_t k_at[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) k_at[k] = column * 256 + (((2 * k + half) ^ (column & 15)) << 4);
+  uint32_t v_at[4];
+  {
+    const int i = lane & 15, g = lane >> 4;
+    const int row = 4 * (g >> 1) + (i >> 2);
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      const int chunk = 4 * d + 2 * (g & 1) + ((i & 3) >> 1);
+      v_at[d] = 2 * kTileBytes + row * 256 + ((chunk ^ (4 * (row & 3))) << 4) + 8 * (i & 1);
+    }
+  }
+
+  v16f o[4];
+#pragma unroll
+  for (int d = 0; d < 4; ++d)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[d][r] = 0.0f;
+  float m = kNegInf, l = 0.0f;
+
+  auto qk = [&](int buffer, v16f (&s)[2]) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[b][r] = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const v8h kf = *reinterpret_cast<const v8h*>(lds + k_at[k] + buffer * kTileBytes + b * 8192);
+        s[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[k], s[b], 0, 0, 0);
+      }
+  };
+  auto softmax = [&](v16f (&s)[2], v8h (&p)[4]) {
+    float mx = s[0][0];
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[b][r]);
+    mx *= a.scale_log2;
+    {
+      const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+      mx = fmaxf(__uint_as_float(x[0]), __uint_as_float(x[1]));
+    }
+    if (__builtin_amdgcn_ballot_w64(mx > m + kRescaleLimit)) {
+      const float m_new = fmaxf(m, mx);
+      const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+      m = m_new;
+      l *= alpha;
+#pragma unroll
+      for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
+    }
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; r += 2) {
+        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[b][r], a.scale_log2, -m));
+        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[b][r + 1], a.scale_log2, -m));
+        l += p0;
+        l += p1;
+        p[2 * b + r / 8][r % 8] = static_cast<_Float16>(p0);
+        p[2 * b + r / 8][r % 8 + 1] = static_cast<_Float16>(p1);
+      }
+  };
+  auto pv = [&](int buffer, v8h (&p)[4]) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        const uint8_t* at = lds + v_at[d] + buffer * kTileBytes + k * 4096;
+        const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((PG_LDS v4s*)at);
+        const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((PG_LDS v4s*)(at + 2048));
+        const v8h vf = __builtin_shufflevector(__builtin_bit_cast(v4h, lo), __builtin_bit_cast(v4h, hi),
+                                               0, 1, 2, 3, 4, 5, 6, 7);
+        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, p[k], o[d], 0, 0, 0);
+      }
+  };
+  auto mask = [&](int tile, v16f (&s)[2]) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int key = tile * kTileKeys + 32 * b + 8 * (r / 4) + 4 * half + r % 4;
+        s[b][r] = key > q ? kNegInf : s[b][r];
+      }
+  };
+  auto barrier = [&]() {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+  };
+  // iteration j: the scores of tile j are in ``s``; K of tile j + 1 and V of
+  // tile j have been requested
+  auto body = [&](int j, int parity, v16f (&s)[2], v16f (&next)[2]) {
+    barrier();
+    if (j + 2 < tiles) load_k(j + 2, parity);
+    load_v(j + 1, parity ^ 1);
+    v8h p[4];
+    qk(parity ^ 1, next);
+    softmax(s, p);
+    pv(parity, p);
+  };
+  auto finish = [&](int j, int parity, v16f (&s)[2]) {
+    barrier();
+    v8h p[4];
+    mask(j, s);
+    softmax(s, p);
+    pv(parity, p);
+  };
+
+  v16f s0[2], s1[2];
+  load_k(0, 0);
+  barrier();
+  if (tiles > 1) load_k(1, 1);
+  load_v(0, 0);
+  qk(0, s0);
+  int j = 0;
+  for (; j + 2 < tiles; j += 2) {
+    body(j, 0, s0, s1);
+    body(j + 1, 1, s1, s0);
+  }
+  if (j + 1 < tiles) {
+    body(j, 0, s0, s1);
+    finish(j + 1, 1, s1);
+  } else {
+    finish(j, 0, s0);
+  }
+
+  {
+    const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
+    l = __uint_as_float(x[0]) + __uint_as_float(x[1]);
+  }
+  if (q >= a.tokens) return;
+  const float inv = 1.0f / l;
+  uint16_t* out = a.out + static_cast<int64_t>(q) * a.out_stride + head * kHeadDim + 4 * half;
+#pragma unroll
+  for (int d = 0; d < 4; ++d)
+#pragma unroll
+    for (int r = 0; r < 16; r += 4) {
+      v4h w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[e] = static_cast<_Float16>(o[d][r + e] * inv);
+      *reinterpret_cast<v4h*>(out + 32 * d + 2 * r) = w;
+    }
+}
+
+// From this many 64-query workgroups on, the 8-wave workgroup, which reads K
+// and V half as often; below it the 4-wave one, whose twice as many workgroups
+// fill the chip.  8 against 4 waves, 8 KV heads: 1024 tokens (128 workgroups)
+// 30.2 against 23.0 us, 2048 54.8 / 49.8, 3072 (384) 90.6 / 91.3, 4096 139 /
+// 153, 16384 1990 / 2124.
+constexpr int64_t kWideBlocks = 384;
+
+template <int kWaves>
+void launch_attention(AttentionArgs a, hipStream_t stream) {
+  constexpr int kQueries = 32 * (kWaves / kGqa);
+  a.blocks = (a.tokens + kQueries - 1) / kQueries;
+  hipLaunchKernelGGL(causal_attention_kernel<kWaves>, dim3(static_cast<unsigned>(a.blocks) * a.kv_heads),
+                     dim3(kWave * kWaves), 0, stream, a);
+}
+
+bool aligned(const void* p, uintptr_t to) { return reinterpret_cast<uintptr_t>(p) % to == 0; }
+
+}  // namespace
+}  // namespace pg
+
+using namespace pg;
+
+extern "C" int32_t pg_causal_attention(const void* query, int64_t query_stride, const void* key,
+                                       int64_t key_stride, const void* value, int64_t value_stride,
+                                       void* out, int64_t out_stride, int32_t tokens,
+                                       int32_t query_heads, int32_t kv_heads, float sm_scale,
+                                       void* stream) {
+  clear_error();
+  if (!query || !key || !value || !out) return fail(PG_ERROR_INVALID_ARGUMENT, "null tensor pointer");
+  if (tokens <= 0) return fail(PG_ERROR_INVALID_ARGUMENT, "the prompt must hold at least one token");
+  if (kv_heads <= 0 || query_heads != kGqa * kv_heads)
+    return fail(PG_ERROR_UNSUPPORTED, "the attention kernel requires GQA group size 4");
+  const int64_t q_row = static_cast<int64_t>(query_heads) * kHeadDim;
+  const int64_t kv_row = static_cast<int64_t>(kv_heads) * kHeadDim;
+  if (query_stride < q_row || out_stride < q_row || key_stride < kv_row || value_stride < kv_row ||
+      query_stride % 8 || key_stride % 8 || value_stride % 8 || out_stride % 4)
+    return fail(PG_ERROR_INVALID_ARGUMENT, "token strides must cover the rows and keep 16-byte alignment");
+  if (!aligned(query, 16) || !aligned(key, 16) || !aligned(value, 16) || !aligned(out, 8))
+    return fail(PG_ERROR_INVALID_ARGUMENT, "attention rows must be 16-byte aligned");
+  if (!(sm_scale > 0.0f) || !__builtin_isfinite(sm_scale))
+    return fail(PG_ERROR_INVALID_ARGUMENT, "sm_scale must be positive and finite");
+  AttentionArgs a{};
+  a.query = static_cast<const uint16_t*>(query);
+  a.key = static_cast<const uint16_t*>(key);
+  a.value = static_cast<const uint16_t*>(value);
+  a.out = static_cast<uint16_t*>(out);
+  a.query_stride = query_stride;
+  a.key_stride = key_stride;
+  a.value_stride = value_stride;
+  a.out_stride = out_stride;
+  a.tokens = tokens;
+  a.kv_heads = kv_heads;
+  a.scale_log2 = sm_scale * 1.4426950408889634f;
+  const int64_t wide = (static_cast<int64_t>(tokens) + 63) / 64 * kv_heads;
+  if (wide >= kWideBlocks) {
+    launch_attention<8>(a, as_stream(stream));
+  } else {
+    launch_attention<4>(a, as_stream(stream));
+  }
+  return check_launch("causal_attention");
+}

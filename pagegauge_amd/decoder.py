@@ -247,13 +247,48 @@ def rope(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
     return x * cos[:, None, :] + rotated * sin[:, None, :]
 
 
+def _on_current_device(*tensors: torch.Tensor) -> bool:
+    """Plain CUDA FP16 tensors of the current device without autograd history
+    (and no tracing): what kernels launched on its current stream may take."""
+    if torch.compiler.is_compiling() or not all(
+            type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda
+            and t.dtype == torch.float16 for t in tensors):
+        return False
+    device = torch.cuda.current_device()
+    return (all(t.get_device() == device for t in tensors)
+            and not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)))
+
+
+def _attention_kernel_takes(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
+    """``pg_causal_attention`` reads FP16 rows of dense [H, 128] heads, 16-byte
+    aligned, of a non-empty prompt with GQA group 4."""
+    return (_on_current_device(q, k, v) and q.shape[0] > 0
+            and q.shape[0] == k.shape[0] == v.shape[0] and k.shape == v.shape
+            and q.shape[1] == GQA * k.shape[1]
+            and all(t.dim() == 3 and t.shape[2] == DIM and t.stride(2) == 1 and t.stride(1) == DIM
+                    and t.stride(0) >= t.shape[1] * DIM and t.stride(0) % 8 == 0
+                    and t.data_ptr() % 16 == 0 for t in (q, k, v)))
+
+
 def _causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                       chunk: int = 1024) -> torch.Tensor:
     """Prefill attention, [T,Hq,128] x [T,Hkv,128] -> [T,Hq,128] FP16.
 
-    Query heads 4g..4g+3 share KV head g, so a block of queries is laid out
-    [Hkv, 4*chunk, 128] and multiplied by contiguous K^T [Hkv, 128, T]; the
-    softmax is float32.  Memory is bounded by the query chunk."""
+    On the GPU one HIP launch (``pg_causal_attention``) where the tensors are
+    laid out as it reads them.  Everything else (the CPU, other types and
+    strides) takes the torch operators: query heads 4g..4g+3 share KV head g,
+    so a block of queries is laid out [Hkv, 4*chunk, 128] and multiplied by
+    contiguous K^T [Hkv, 128, T]; the softmax is float32.  Memory is bounded
+    by the query chunk."""
+    if _attention_kernel_takes(q, k, v):
+        from . import _capi
+
+        out = torch.empty(q.shape, device=q.device, dtype=q.dtype)
+        _capi.call("pg_causal_attention", q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0),
+                   v.data_ptr(), v.stride(0), out.data_ptr(), out.stride(0), int(q.shape[0]),
+                   int(q.shape[1]), int(k.shape[1]), 1.0 / math.sqrt(DIM),
+                   torch.cuda.current_stream().cuda_stream)
+        return out
     tokens, hq, _ = q.shape
     hkv = k.shape[1]
     scale = 1.0 / math.sqrt(DIM)
