@@ -234,6 +234,29 @@ int32_t pg_causal_attention(const void* query, int64_t query_stride, const void*
                             void* out, int64_t out_stride, int32_t tokens, int32_t query_heads,
                             int32_t kv_heads, float sm_scale, void* stream);
 
+/* The element-wise work between the GEMMs of a prompt's decoder layers
+ * (rms_norm, rope, SiLU * up and the residual adds of
+ * scripts/benchmark_page_gauge_transformer.py's TransformerDecoder), rounded
+ * where FP16 torch operators round.  All rows fp16, 16-byte aligned, strides
+ * multiples of 8 elements.
+ *
+ * pg_rms_norm: with delta, x += delta in place first (one FP16 add); then
+ * out = weight * fp16(x * rsqrt(mean(x^2) + eps)), float32 statistics, per
+ * row of ``width`` elements (a multiple of 8, at most 16384).
+ * pg_rope_rows: token t's query_heads + kv_heads leading head rows of qkv,
+ * rotated by row t of the [tokens, 128] tables, into dense query [tokens,
+ * query_heads, 128] and key [tokens, kv_heads, 128].
+ * pg_swiglu: out = silu(gate) * up of rows [gate | up] of 2 * width
+ * elements (width a multiple of 8). */
+int32_t pg_rms_norm(void* x, int64_t x_stride, const void* delta, int64_t delta_stride,
+                    const void* weight, float eps, void* out, int64_t out_stride, int64_t rows,
+                    int32_t width, void* stream);
+int32_t pg_rope_rows(const void* qkv, int64_t qkv_stride, const void* cosine, const void* sine,
+                     int64_t rope_stride, void* query, void* key, int64_t tokens,
+                     int32_t query_heads, int32_t kv_heads, void* stream);
+int32_t pg_swiglu(const void* gate_up, int64_t stride, void* out, int64_t out_stride,
+                  int64_t rows, int32_t width, void* stream);
+
 /* ------------------------------------------------------------------------
  * Paged decode (K1) and the split scheduler (S).
  * ---------------------------------------------------------------------- */

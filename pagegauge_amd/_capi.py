@@ -84,6 +84,9 @@ PROTOTYPES = {
     "pg_token_major_centers_noalloc": (_i32, [_p, _i64, _p, _i64, _i64, _i32, _p, _p, _p]),
     "pg_causal_attention": (_i32, [_p, _i64, _p, _i64, _p, _i64, _p, _i64, _i32, _i32, _i32, _f32,
                                    _p]),
+    "pg_rms_norm": (_i32, [_p, _i64, _p, _i64, _p, _f32, _p, _i64, _i64, _i32, _p]),
+    "pg_rope_rows": (_i32, [_p, _i64, _p, _p, _i64, _p, _p, _i64, _i32, _i32, _p]),
+    "pg_swiglu": (_i32, [_p, _i64, _p, _i64, _i64, _i32, _p]),
     "pg_decode_workspace_bytes": (_i64, [_i32, _i32, _i64, _i64]),
     "pg_select_split_pages": (_i32, [_i64, _i32, _i32, _i32, _i32]),
     "pg_decode_plan": (_i32, [_p, _p, _i32, _i32, _p, _p, _i32, _i32, _i32, _i32, _i32, _i32,

@@ -309,6 +309,100 @@ def _causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     return out
 
 
+def _prefill_kernels_take(weights: DecoderWeights, tokens: torch.Tensor, cos: torch.Tensor,
+                          sin: torch.Tensor) -> bool:
+    """Whether ``prefill`` runs its element-wise work as HIP kernels: FP16
+    weights and dense 16-byte aligned RoPE rows on the current device, widths
+    that the kernels read (multiples of 8; norms up to 16384).  The GEMMs'
+    inputs and outputs are fresh tensors, dense and aligned."""
+    cfg = weights.config
+    return (tokens.numel() > 0 and cfg.hidden % 8 == 0 and cfg.hidden <= 16384
+            and cfg.intermediate % 8 == 0 and tokens.numel() <= min(cos.shape[0], sin.shape[0])
+            and _on_current_device(weights.embed, weights.norm, weights.lm_head, cos, sin,
+                                   *(w for layer in weights.layers for w in layer.values()))
+            and tokens.device == weights.embed.device
+            and all(t.dim() == 2 and t.shape[1] == DIM and t.stride(1) == 1
+                    and t.stride(0) % 8 == 0 and t.stride(0) >= DIM and t.data_ptr() % 16 == 0
+                    for t in (cos, sin))
+            and cos.stride(0) == sin.stride(0)
+            and all(t.is_contiguous() and t.data_ptr() % 16 == 0
+                    for layer in weights.layers for t in (layer["input_norm"], layer["post_norm"])))
+
+
+def _norm_rows(x: torch.Tensor, weight: torch.Tensor, eps: float,
+               delta: Optional[torch.Tensor]) -> torch.Tensor:
+    """``rms_norm(x + delta)``, the sum left in ``x``, in one HIP launch."""
+    from . import _capi
+
+    out = torch.empty_like(x)
+    _capi.call("pg_rms_norm", x.data_ptr(), x.stride(0), None if delta is None else delta.data_ptr(),
+               0 if delta is None else delta.stride(0), weight.data_ptr(), float(eps),
+               out.data_ptr(), out.stride(0), int(x.shape[0]), int(x.shape[1]),
+               torch.cuda.current_stream().cuda_stream)
+    return out
+
+
+def _rope_rows(cfg: DecoderConfig, qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor):
+    """``rope`` of the query and key rows of a fused QKV projection (one HIP launch)."""
+    from . import _capi
+
+    count = int(qkv.shape[0])
+    q = torch.empty(count, cfg.q_heads, DIM, device=qkv.device, dtype=qkv.dtype)
+    k = torch.empty(count, cfg.kv_heads, DIM, device=qkv.device, dtype=qkv.dtype)
+    _capi.call("pg_rope_rows", qkv.data_ptr(), qkv.stride(0), cos.data_ptr(), sin.data_ptr(),
+               cos.stride(0), q.data_ptr(), k.data_ptr(), count, cfg.q_heads, cfg.kv_heads,
+               torch.cuda.current_stream().cuda_stream)
+    return q, k
+
+
+def _swiglu_rows(gate_up: torch.Tensor) -> torch.Tensor:
+    """``F.silu(gate) * up`` of rows [gate | up] (one HIP launch)."""
+    from . import _capi
+
+    rows, width = int(gate_up.shape[0]), int(gate_up.shape[1]) // 2
+    out = torch.empty(rows, width, device=gate_up.device, dtype=gate_up.dtype)
+    _capi.call("pg_swiglu", gate_up.data_ptr(), gate_up.stride(0), out.data_ptr(), out.stride(0),
+               rows, width, torch.cuda.current_stream().cuda_stream)
+    return out
+
+
+def _prefill_layers(weights: DecoderWeights, hidden: torch.Tensor, cos: torch.Tensor,
+                    sin: torch.Tensor, on_layer) -> torch.Tensor:
+    """The layers of ``prefill`` on ``hidden`` [T, hidden] in place, the
+    element-wise work as HIP kernels: each residual add is left to the norm
+    that follows it.  Same roundings as the torch operators.  Returns the last
+    token's row [1, hidden] (a prompt's logits need no other)."""
+    cfg = weights.config
+    count = int(hidden.shape[0])
+    qw, kw = cfg.q_heads * DIM, cfg.kv_heads * DIM
+    delta = None
+    for index, w in enumerate(weights.layers):
+        qkv = F.linear(_norm_rows(hidden, w["input_norm"], cfg.rms_eps, delta), w["qkv"])
+        q, k = _rope_rows(cfg, qkv, cos, sin)
+        v = qkv[:, qw + kw:].view(count, cfg.kv_heads, DIM)
+        if on_layer is not None:
+            on_layer(index, k, v)
+        attn = _causal_attention(q, k, v)
+        delta = F.linear(attn.reshape(count, qw), w["o"])
+        del qkv, q, k, v, attn
+        gate_up = F.linear(_norm_rows(hidden, w["post_norm"], cfg.rms_eps, delta), w["gate_up"])
+        delta = F.linear(_swiglu_rows(gate_up), w["down"])
+        del gate_up
+    return hidden[-1:] if delta is None else hidden[-1:] + delta[-1:]
+
+
+def _head_rows(weights: DecoderWeights, last: torch.Tensor) -> torch.Tensor:
+    """Final norm and LM head of one row: float32 logits [1, vocab], one launch
+    of the decode step's projection where its width allows (multiples of 512
+    up to 32768: 43 against 91 us as norm, GEMM and cast at 4096 x 32768)."""
+    cfg = weights.config
+    if cfg.hidden % 512 or cfg.hidden > 32768 or not all(
+            w.is_contiguous() and w.data_ptr() % 16 == 0 for w in (weights.lm_head, weights.norm)):
+        return F.linear(rms_norm(last, weights.norm, cfg.rms_eps), weights.lm_head).float()
+    logits = torch.empty(1, weights.lm_head.shape[0], device=last.device, dtype=torch.float32)
+    return projection(weights.lm_head, last, logits, norm_weight=weights.norm, eps=cfg.rms_eps)
+
+
 @torch.inference_mode()
 def prefill(weights: DecoderWeights, tokens: torch.Tensor, cos: torch.Tensor,
             sin: torch.Tensor, on_layer=None) -> torch.Tensor:
@@ -321,6 +415,8 @@ def prefill(weights: DecoderWeights, tokens: torch.Tensor, cos: torch.Tensor,
     count = tokens.numel()
     hidden = F.embedding(tokens, weights.embed)
     c, s = cos[:count], sin[:count]
+    if _prefill_kernels_take(weights, tokens, cos, sin):
+        return _head_rows(weights, _prefill_layers(weights, hidden, c, s, on_layer))
     qw, kw = cfg.q_heads * DIM, cfg.kv_heads * DIM
     for index, w in enumerate(weights.layers):
         x = rms_norm(hidden, w["input_norm"], cfg.rms_eps)
