@@ -187,6 +187,20 @@ int32_t pg_prefill_page_gauge(const void* key, int64_t key_token_stride, const v
                               void* exact_value_pages, int64_t num_pages, int32_t heads,
                               void* stream);
 
+/* pg_prefill_page_gauge with the exact pages given by the cache layout of the
+ * decoder (a builder addition: the reference builds the map on the host).
+ * Logical page p of the num_pages pages is also written, centered, to exact
+ * page first_slot + p if p < sink_pages; first_slot + sink_pages + p -
+ * suffix_begin if it is one of the suffix_pages pages from suffix_begin on;
+ * first_slot + sink_pages + suffix_pages + p % tail_pages if it is one of the
+ * last tail_pages (> 0) pages.  num_exact_pages bounds the exact pool. */
+int32_t pg_prefill_page_gauge_layout(
+    const void* key, int64_t key_token_stride, const void* value, int64_t value_token_stride,
+    const void* key_center, const void* value_center, int8_t* key_codes, int8_t* value_codes,
+    void* key_scales, void* value_scales, void* exact_key_pages, void* exact_value_pages,
+    int64_t num_exact_pages, int64_t first_slot, int32_t sink_pages, int32_t suffix_begin,
+    int32_t suffix_pages, int32_t tail_pages, int64_t num_pages, int32_t heads, void* stream);
+
 /* Per-(head, dim) channel centers of a token-major K/V prefix: replaces
  * token_major_centers (diagnostics/benchmark_backend_exclusive.py:372-395) and
  * the center lines of build_caches (scripts/benchmark_page_gauge_transformer.py:1201-1214),

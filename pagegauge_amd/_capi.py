@@ -78,6 +78,8 @@ PROTOTYPES = {
     "pg_quantize_page_gauge": (_i32, [_p, _p, _p, _p, _i64, _i32, _p]),
     "pg_prefill_page_gauge": (_i32, [_p, _i64, _p, _i64, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64,
                                      _i32, _p]),
+    "pg_prefill_page_gauge_layout": (_i32, [_p, _i64, _p, _i64, _p, _p, _p, _p, _p, _p, _p, _p,
+                                            _i64, _i64, _i32, _i32, _i32, _i32, _i64, _i32, _p]),
     "pg_token_major_centers_workspace_bytes": (_i64, [_i64, _i32]),
     "pg_token_major_centers": (_i32, [_p, _i64, _p, _i64, _i64, _i32, _p, _p, _p, _i64, _p]),
     "pg_token_major_centers_noalloc_max_bytes": (_i64, []),

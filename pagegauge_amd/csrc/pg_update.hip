@@ -109,15 +109,10 @@ __device__ __forceinline__ uint16_t centered(uint16_t a, uint16_t b) {
   return __half_as_ushort(__float2half_rn(diff));
 }
 
+// sign * floor(|quotient| + 0.5), clamped to [-127, 127]; a NaN gives 0.
 __device__ __forceinline__ int8_t sign_symmetric_code(float quotient) {
-  int code;
-  if (quotient >= 0.0f) {
-    code = static_cast<int>(floorf(quotient + 0.5f));
-  } else {
-    code = -static_cast<int>(floorf(-quotient + 0.5f));
-  }
-  code = max(-127, min(127, code));
-  return static_cast<int8_t>(code);
+  const float rounded = __builtin_copysignf(floorf(fabsf(quotient) + 0.5f), quotient);
+  return static_cast<int8_t>(max(-127, min(127, static_cast<int>(rounded))));
 }
 
 __device__ __forceinline__ uint16_t stored_scale(float maximum) {
@@ -322,6 +317,13 @@ struct QuantizeParams {
   uint16_t* exact_key;
   uint16_t* exact_value;
   int half_even;
+  // Without a map, tail_pages > 0: the slots of a request's exact layout
+  // (prefix, static suffix and tail ring from first_slot on).
+  int64_t first_slot;
+  int sink_pages;
+  int suffix_begin;
+  int suffix_pages;
+  int tail_pages;
 };
 
 // Round-half-even of the quotient (v_rndne_f32 under the default rounding
@@ -369,6 +371,20 @@ __device__ __forceinline__ void quantize_block(const uint16_t* src, int64_t src_
   }
 }
 
+// Exact slot of logical page ``page``: the explicit map's entry, or the
+// layout's (prefix, static suffix, tail ring); -1 for a page with codes only.
+__device__ __forceinline__ int64_t exact_slot(const QuantizeParams& p, int64_t page) {
+  if (p.exact_map != nullptr) return p.exact_map[page];
+  if (p.tail_pages <= 0) return -1;
+  if (page < p.sink_pages) return p.first_slot + page;
+  if (page >= p.suffix_begin && page < p.suffix_begin + p.suffix_pages)
+    return p.first_slot + p.sink_pages + (page - p.suffix_begin);
+  if (page >= p.num_pages - p.tail_pages)
+    return p.first_slot + p.sink_pages + p.suffix_pages + page % p.tail_pages;
+  return -1;
+}
+
+// Any alignment of the rows: one wave per (page, head), 4-byte accesses.
 __global__ __launch_bounds__(kWave * kWavesPerBlock) void quantize_pages_kernel(QuantizeParams p) {
   const int lane = threadIdx.x % kWave;
   const int64_t item = static_cast<int64_t>(blockIdx.x) * kWavesPerBlock + threadIdx.x / kWave;
@@ -377,8 +393,8 @@ __global__ __launch_bounds__(kWave * kWavesPerBlock) void quantize_pages_kernel(
   const int head = static_cast<int>(item % p.heads);
   const int64_t row_stride = static_cast<int64_t>(p.heads) * kHeadDim;
   const int64_t base = (page * kPageSize * p.heads + head) * kHeadDim;
-  const int32_t ring_page = p.exact_map != nullptr ? p.exact_map[page] : -1;
-  const int64_t ring_base = (static_cast<int64_t>(ring_page) * kPageSize * p.heads + head) * kHeadDim;
+  const int64_t ring_page = exact_slot(p, page);
+  const int64_t ring_base = (ring_page * kPageSize * p.heads + head) * kHeadDim;
   quantize_block(p.key + page * kPageSize * p.key_token_stride + head * kHeadDim,
                  p.key_token_stride, p.key_center + head * kHeadDim, row_stride,
                  p.key_codes + base, p.key_scales + item,
@@ -388,6 +404,122 @@ __global__ __launch_bounds__(kWave * kWavesPerBlock) void quantize_pages_kernel(
                    p.value_token_stride, p.value_center + head * kHeadDim, row_stride,
                    p.value_codes + base, p.value_scales + item,
                    ring_page >= 0 ? p.exact_value + ring_base : nullptr, lane, p.half_even != 0);
+}
+
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+
+// One (page, head) block of 16 rows from registers: lane (r, c) of 4 x 16
+// holds dims 8c..8c+7 of rows r, r + 4, r + 8, r + 12 (``rows``).
+//
+// The quotient x / scale is the IEEE one, by three operations instead of a
+// division: with r = RN(1 / scale), q0 = RN(x * r) is within 2 ulp of it, the
+// residual e = x - q0 * scale is exact (the scale has the 11 bits of an FP16
+// value, and x, the difference of two FP16 values in float32, lies far from
+// float32's limits), and q = RN(q0 + e * r) adds e / scale with a relative
+// error of 2^-24, that is within 2^-23 ulp of the true quotient before its
+// rounding.  A quotient of a 24-bit by an 11-bit number is never a midpoint
+// of two floats and lies at least 2^-12 ulp from one, so q is correctly
+// rounded.  An infinite scale (infinite or NaN input) takes the division.
+__device__ __forceinline__ void quantize_rows(const v4u (&rows)[4], v4u center, int64_t row_stride,
+                                              int8_t* codes, uint16_t* scale_out, uint16_t* ring,
+                                              int lane, bool half_even) {
+  float c[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    c[e] = half_bits_to_float(static_cast<uint16_t>(center[e >> 1] >> (16 * (e & 1))));
+  float x[4][8];
+  float local_max = 0.0f;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      x[t][e] = half_bits_to_float(static_cast<uint16_t>(rows[t][e >> 1] >> (16 * (e & 1)))) - c[e];
+      local_max = fmaxf(local_max, fabsf(x[t][e]));
+    }
+  }
+  local_max = row16_max(local_max);
+  local_max = fmaxf(local_max, __shfl_xor(local_max, 16, kWave));
+  local_max = fmaxf(local_max, __shfl_xor(local_max, 32, kWave));
+  const int64_t at = (lane >> 4) * row_stride + 8 * (lane & 15);
+  if (ring != nullptr) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      v4u w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        w[e] = static_cast<uint32_t>(__half_as_ushort(__float2half_rn(x[t][2 * e]))) |
+               static_cast<uint32_t>(__half_as_ushort(__float2half_rn(x[t][2 * e + 1]))) << 16;
+      *reinterpret_cast<v4u*>(ring + at + 4 * t * row_stride) = w;
+    }
+  }
+  // the scale is the same in every lane: a scalar, so that the branch below is one
+  const uint16_t scale_bits = static_cast<uint16_t>(
+      __builtin_amdgcn_readfirstlane(static_cast<int>(stored_scale(local_max))));
+  if (lane == 0) *scale_out = scale_bits;
+  const float scale = half_bits_to_float(scale_bits);
+  const bool finite = scale_bits < 0x7c00u;
+  const float inverse = 1.0f / scale;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    int code[8];
+    if (finite) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float q0 = x[t][e] * inverse;
+        const float q = __builtin_fmaf(__builtin_fmaf(-q0, scale, x[t][e]), inverse, q0);
+        code[e] = half_even ? half_even_code(q) : sign_symmetric_code(q);
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float q = x[t][e] / scale;
+        code[e] = half_even ? half_even_code(q) : sign_symmetric_code(q);
+      }
+    }
+    v2u w;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      // byte 0 of four codes
+      const uint32_t lo = __builtin_amdgcn_perm(code[4 * e + 1], code[4 * e], 0x0c0c0400u);
+      const uint32_t hi = __builtin_amdgcn_perm(code[4 * e + 3], code[4 * e + 2], 0x04000c0cu);
+      w[e] = lo | hi;
+    }
+    *reinterpret_cast<v2u*>(codes + at + 4 * t * row_stride) = w;
+  }
+}
+
+// Rows of 16-byte aligned 8-dim vectors: one wave per (page, head, tensor),
+// 16-byte loads (4 rows per instruction, the block's four requested before
+// the first is used), 8-byte code stores and no division: bound by HBM.
+// 16384 tokens x 8 heads, K and V (101 MB): 36.3 us with 4-byte accesses and
+// divisions, 33.8 with both tensors in one wave and a per-lane branch around
+// the division, 20.8 (4.9 TB/s) like this.
+// Grid (blocks of 4 waves, 1 or 2 tensors).  kHalfEven: the rounding of
+// quantize_page_gauge.
+template <bool kHalfEven>
+__global__ __launch_bounds__(kWave * kWavesPerBlock) void quantize_pages_wide_kernel(QuantizeParams p) {
+  const int lane = threadIdx.x % kWave;
+  const int64_t item = static_cast<int64_t>(blockIdx.x) * kWavesPerBlock + threadIdx.x / kWave;
+  if (item >= p.num_pages * p.heads) return;
+  const bool second = blockIdx.y != 0;
+  const int64_t page = item / p.heads;
+  const int head = static_cast<int>(item - page * p.heads);
+  const int column = head * kHeadDim + 8 * (lane & 15);
+  const int64_t stride = second ? p.value_token_stride : p.key_token_stride;
+  const uint16_t* src = (second ? p.value : p.key) + (page * kPageSize + (lane >> 4)) * stride + column;
+  v4u rows[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) rows[t] = *reinterpret_cast<const v4u*>(src + 4 * t * stride);
+  const v4u center = *reinterpret_cast<const v4u*>((second ? p.value_center : p.key_center) + column);
+  const int64_t row_stride = static_cast<int64_t>(p.heads) * kHeadDim;
+  const int64_t base = (page * kPageSize * p.heads + head) * kHeadDim;
+  const int64_t ring_page = exact_slot(p, page);
+  uint16_t* ring = ring_page >= 0 ? (second ? p.exact_value : p.exact_key) +
+                                        (ring_page * kPageSize * p.heads + head) * kHeadDim
+                                  : nullptr;
+  quantize_rows(rows, center, row_stride, (second ? p.value_codes : p.key_codes) + base,
+                (second ? p.value_scales : p.key_scales) + item, ring, lane, kHalfEven);
 }
 
 // Exact per-(head, dim) token mean.  Every FP16 value is an integer multiple
@@ -472,8 +604,27 @@ int32_t launch_quantize(const QuantizeParams& p, hipStream_t stream, const char*
   const int64_t waves = p.num_pages * p.heads;
   const int64_t blocks = (waves + kWavesPerBlock - 1) / kWavesPerBlock;
   if (blocks > 0x7fffffff) return fail(PG_ERROR_INVALID_ARGUMENT, "too many pages");
-  hipLaunchKernelGGL(quantize_pages_kernel, dim3(static_cast<unsigned>(blocks)),
-                     dim3(kWave * kWavesPerBlock), 0, stream, p);
+  const auto aligned = [](const void* q, uintptr_t to) { return reinterpret_cast<uintptr_t>(q) % to == 0; };
+  // null pointers (one tensor, no ring) are aligned; rows of heads * 128
+  // elements keep the alignment of their base
+  const bool wide = p.key_token_stride % 8 == 0 && p.value_token_stride % 8 == 0 &&
+                    aligned(p.key, 16) && aligned(p.value, 16) && aligned(p.key_center, 16) &&
+                    aligned(p.value_center, 16) && aligned(p.key_codes, 8) &&
+                    aligned(p.value_codes, 8) && aligned(p.exact_key, 16) &&
+                    aligned(p.exact_value, 16);
+  if (wide) {
+    const dim3 grid(static_cast<unsigned>(blocks), p.value != nullptr ? 2 : 1);
+    if (p.half_even) {
+      hipLaunchKernelGGL(quantize_pages_wide_kernel<true>, grid, dim3(kWave * kWavesPerBlock), 0,
+                         stream, p);
+    } else {
+      hipLaunchKernelGGL(quantize_pages_wide_kernel<false>, grid, dim3(kWave * kWavesPerBlock), 0,
+                         stream, p);
+    }
+  } else {
+    hipLaunchKernelGGL(quantize_pages_kernel, dim3(static_cast<unsigned>(blocks)),
+                       dim3(kWave * kWavesPerBlock), 0, stream, p);
+  }
   return check_launch(what);
 }
 
@@ -805,28 +956,24 @@ extern "C" int32_t pg_quantize_page_gauge(const void* values, const void* center
   return launch_quantize(p, as_stream(stream), "quantize_page_gauge");
 }
 
-extern "C" int32_t pg_prefill_page_gauge(const void* key, int64_t key_token_stride,
-                                         const void* value, int64_t value_token_stride,
-                                         const void* key_center, const void* value_center,
-                                         int8_t* key_codes, int8_t* value_codes,
-                                         void* key_scales, void* value_scales,
-                                         const int32_t* exact_page_map, void* exact_key_pages,
-                                         void* exact_value_pages, int64_t num_pages,
-                                         int32_t heads, void* stream) {
-  clear_error();
+namespace {
+
+// Checks and the parameters without the exact pages of both prefill entry points.
+int32_t prefill_params(const void* key, int64_t key_token_stride, const void* value,
+                       int64_t value_token_stride, const void* key_center,
+                       const void* value_center, int8_t* key_codes, int8_t* value_codes,
+                       void* key_scales, void* value_scales, int64_t num_pages, int32_t heads,
+                       QuantizeParams& p) {
   if (num_pages <= 0 || heads <= 0)
     return fail(PG_ERROR_INVALID_ARGUMENT, "pages and heads must be positive");
   if (any_null({key, value, key_center, value_center, key_codes, value_codes, key_scales,
                 value_scales}))
     return fail(PG_ERROR_INVALID_ARGUMENT, "null tensor pointer");
-  if (exact_page_map != nullptr && (exact_key_pages == nullptr || exact_value_pages == nullptr))
-    return fail(PG_ERROR_INVALID_ARGUMENT, "an exact page map needs exact key/value pages");
   const int64_t row = static_cast<int64_t>(heads) * kHeadDim;
   if (key_token_stride < row || value_token_stride < row || key_token_stride % 2 ||
       value_token_stride % 2)
     return fail(PG_ERROR_INVALID_ARGUMENT,
                 "token strides must be even and cover heads*128 elements");
-  QuantizeParams p{};
   p.key = static_cast<const uint16_t*>(key);
   p.value = static_cast<const uint16_t*>(value);
   p.key_center = static_cast<const uint16_t*>(key_center);
@@ -839,10 +986,62 @@ extern "C" int32_t pg_prefill_page_gauge(const void* key, int64_t key_token_stri
   p.heads = heads;
   p.key_token_stride = key_token_stride;
   p.value_token_stride = value_token_stride;
+  return PG_OK;
+}
+
+}  // namespace
+
+extern "C" int32_t pg_prefill_page_gauge(const void* key, int64_t key_token_stride,
+                                         const void* value, int64_t value_token_stride,
+                                         const void* key_center, const void* value_center,
+                                         int8_t* key_codes, int8_t* value_codes,
+                                         void* key_scales, void* value_scales,
+                                         const int32_t* exact_page_map, void* exact_key_pages,
+                                         void* exact_value_pages, int64_t num_pages,
+                                         int32_t heads, void* stream) {
+  clear_error();
+  QuantizeParams p{};
+  if (int32_t rc = prefill_params(key, key_token_stride, value, value_token_stride, key_center,
+                                  value_center, key_codes, value_codes, key_scales, value_scales,
+                                  num_pages, heads, p))
+    return rc;
+  if (exact_page_map != nullptr && (exact_key_pages == nullptr || exact_value_pages == nullptr))
+    return fail(PG_ERROR_INVALID_ARGUMENT, "an exact page map needs exact key/value pages");
   p.exact_map = exact_page_map;
   p.exact_key = static_cast<uint16_t*>(exact_key_pages);
   p.exact_value = static_cast<uint16_t*>(exact_value_pages);
   return launch_quantize(p, as_stream(stream), "prefill_page_gauge");
+}
+
+extern "C" int32_t pg_prefill_page_gauge_layout(
+    const void* key, int64_t key_token_stride, const void* value, int64_t value_token_stride,
+    const void* key_center, const void* value_center, int8_t* key_codes, int8_t* value_codes,
+    void* key_scales, void* value_scales, void* exact_key_pages, void* exact_value_pages,
+    int64_t num_exact_pages, int64_t first_slot, int32_t sink_pages, int32_t suffix_begin,
+    int32_t suffix_pages, int32_t tail_pages, int64_t num_pages, int32_t heads, void* stream) {
+  clear_error();
+  if (!exact_key_pages || !exact_value_pages)
+    return fail(PG_ERROR_INVALID_ARGUMENT, "null tensor pointer");
+  if (sink_pages < 0 || suffix_begin < 0 || suffix_pages < 0 || tail_pages <= 0 || first_slot < 0)
+    return fail(PG_ERROR_INVALID_ARGUMENT,
+                "the exact layout needs non-negative fixed pages and a tail ring");
+  if (suffix_pages > 0 && suffix_begin < sink_pages)
+    return fail(PG_ERROR_INVALID_ARGUMENT, "the static suffix must lie behind the prefix");
+  if (first_slot + sink_pages + suffix_pages + tail_pages > num_exact_pages)
+    return fail(PG_ERROR_INVALID_ARGUMENT, "the exact layout points past the exact pages");
+  QuantizeParams p{};
+  if (int32_t rc = prefill_params(key, key_token_stride, value, value_token_stride, key_center,
+                                  value_center, key_codes, value_codes, key_scales, value_scales,
+                                  num_pages, heads, p))
+    return rc;
+  p.exact_key = static_cast<uint16_t*>(exact_key_pages);
+  p.exact_value = static_cast<uint16_t*>(exact_value_pages);
+  p.first_slot = first_slot;
+  p.sink_pages = sink_pages;
+  p.suffix_begin = suffix_begin;
+  p.suffix_pages = suffix_pages;
+  p.tail_pages = tail_pages;
+  return launch_quantize(p, as_stream(stream), "prefill_page_gauge_layout");
 }
 
 extern "C" int64_t pg_token_major_centers_workspace_bytes(int64_t tokens, int32_t heads) {

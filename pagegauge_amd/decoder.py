@@ -41,7 +41,7 @@ from . import page_table as pt
 from .decode import (BatchDecodeWithPagedKVCacheWrapper, HeterogeneousDecodeWrapper,
                      PageGaugeSegmentedDecode)
 from .runtime import load_append_extension
-from .update import prefill_page_gauge, token_major_centers
+from .update import prefill_page_gauge_layout, token_major_centers
 
 PAGE = 16
 DIM = 128
@@ -527,21 +527,15 @@ class GaugeCache:
             self._center_workspace = torch.empty(need, device=key.device, dtype=torch.uint8)
         kc, vc = self.key_center[layer, request], self.value_center[layer, request]
         token_major_centers(key, value, kc, vc, self._center_workspace)
-        exact_map = torch.full((pages,), -1, dtype=torch.int32)
-        partition = pt.page_gauge_logical_partition(
-            pages, self.exact_tail_pages, self.exact_sink_pages, PAGE,
-            self.exact_static_suffix_pages, self.initial_context_pages)
-        for logical in partition["exact_logical_pages"]:
-            exact_map[logical] = pt.exact_physical_page_index(
-                request, logical, self.exact_tail_pages, self.exact_sink_pages,
-                self.exact_static_suffix_pages, self.initial_context_pages)
+        layout = pt.ExactPageLayout.checked(self.exact_sink_pages, self.exact_static_suffix_pages,
+                                            self.initial_context_pages, self.exact_tail_pages)
         base = request * self.pages_per_request
-        prefill_page_gauge(key, value, kc, vc,
-                           self.key_codes[layer, base:base + pages],
-                           self.value_codes[layer, base:base + pages],
-                           self.key_scales[layer, base:base + pages],
-                           self.value_scales[layer, base:base + pages],
-                           exact_map.to(key.device), self.exact_key[layer], self.exact_value[layer])
+        prefill_page_gauge_layout(key, value, kc, vc,
+                                  self.key_codes[layer, base:base + pages],
+                                  self.value_codes[layer, base:base + pages],
+                                  self.key_scales[layer, base:base + pages],
+                                  self.value_scales[layer, base:base + pages],
+                                  self.exact_key[layer], self.exact_value[layer], request, layout)
 
 
 # ---------------------------------------------------------------------------

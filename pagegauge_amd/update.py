@@ -183,22 +183,9 @@ def token_major_centers(source_key: torch.Tensor, source_value: torch.Tensor,
     return key_center, value_center
 
 
-def prefill_page_gauge(source_key: torch.Tensor, source_value: torch.Tensor,
-                       key_center: torch.Tensor, value_center: torch.Tensor,
-                       key_codes: torch.Tensor, value_codes: torch.Tensor,
-                       key_scales: torch.Tensor, value_scales: torch.Tensor,
-                       exact_page_map: torch.Tensor | None = None,
-                       exact_key_pages: torch.Tensor | None = None,
-                       exact_value_pages: torch.Tensor | None = None) -> None:
-    """Quantise a token-major prefix into INT8 pages and store its exact pages.
-
-    Mirrors the cache population of ``populate_backend_cache_layer``
-    (diagnostics/benchmark_backend_exclusive.py:442-506): every page gets
-    codes and scales from float32-centered values (``quantize_completed_kv_pages``
-    arithmetic) and page ``i`` with ``exact_page_map[i] >= 0`` is also written
-    as ``fp16(f32(x) - f32(center))`` into that ring page.  ``source_*`` are
-    [pages*16, Hkv, 128] FP16 (token rows may be strided).
-    """
+def _prefill_source_checks(source_key, source_value, key_center, value_center, key_codes,
+                           value_codes, key_scales, value_scales) -> tuple[int, int, int, int]:
+    """(pages, heads, key token stride, value token stride) of a prefix."""
     if source_key.shape != source_value.shape or source_key.ndim != 3:
         raise ValueError("token-major K/V must have identical [T,Hkv,D] shapes")
     tokens, heads = int(source_key.shape[0]), int(source_key.shape[1])
@@ -216,15 +203,41 @@ def prefill_page_gauge(source_key: torch.Tensor, source_value: torch.Tensor,
             raise ValueError("scales must be float16 [pages,heads]")
     _all_cuda_contiguous(key_center, value_center, key_codes, value_codes, key_scales,
                          value_scales)
+    return pages, heads, key_stride, value_stride
+
+
+def _exact_page_checks(heads, exact_key_pages, exact_value_pages) -> None:
+    for ring in (exact_key_pages, exact_value_pages):
+        if ring.dtype != torch.float16 or ring.ndim != 4 or tuple(ring.shape[1:]) != (PAGE, heads, DIM):
+            raise ValueError("exact pages must be float16 [ring_pages,16,heads,128]")
+
+
+def prefill_page_gauge(source_key: torch.Tensor, source_value: torch.Tensor,
+                       key_center: torch.Tensor, value_center: torch.Tensor,
+                       key_codes: torch.Tensor, value_codes: torch.Tensor,
+                       key_scales: torch.Tensor, value_scales: torch.Tensor,
+                       exact_page_map: torch.Tensor | None = None,
+                       exact_key_pages: torch.Tensor | None = None,
+                       exact_value_pages: torch.Tensor | None = None) -> None:
+    """Quantise a token-major prefix into INT8 pages and store its exact pages.
+
+    Mirrors the cache population of ``populate_backend_cache_layer``
+    (diagnostics/benchmark_backend_exclusive.py:442-506): every page gets
+    codes and scales from float32-centered values (``quantize_completed_kv_pages``
+    arithmetic) and page ``i`` with ``exact_page_map[i] >= 0`` is also written
+    as ``fp16(f32(x) - f32(center))`` into that ring page.  ``source_*`` are
+    [pages*16, Hkv, 128] FP16 (token rows may be strided).
+    """
+    pages, heads, key_stride, value_stride = _prefill_source_checks(
+        source_key, source_value, key_center, value_center, key_codes, value_codes, key_scales,
+        value_scales)
     map_ptr = ring_k = ring_v = None
     if exact_page_map is not None:
         if exact_page_map.dtype != torch.int32 or tuple(exact_page_map.shape) != (pages,):
             raise ValueError("exact_page_map must be int32 [pages]")
         if exact_key_pages is None or exact_value_pages is None:
             raise ValueError("an exact page map needs exact key/value pages")
-        for ring in (exact_key_pages, exact_value_pages):
-            if ring.dtype != torch.float16 or ring.ndim != 4 or tuple(ring.shape[1:]) != (PAGE, heads, DIM):
-                raise ValueError("exact pages must be float16 [ring_pages,16,heads,128]")
+        _exact_page_checks(heads, exact_key_pages, exact_value_pages)
         _all_cuda_contiguous(exact_page_map, exact_key_pages, exact_value_pages)
         valid = exact_page_map[exact_page_map >= 0]
         if valid.numel() and int(valid.max()) >= exact_key_pages.shape[0]:
@@ -235,3 +248,30 @@ def prefill_page_gauge(source_key: torch.Tensor, source_value: torch.Tensor,
                value_stride, key_center.data_ptr(), value_center.data_ptr(), key_codes.data_ptr(),
                value_codes.data_ptr(), key_scales.data_ptr(), value_scales.data_ptr(), map_ptr,
                ring_k, ring_v, pages, heads, _stream())
+
+
+def prefill_page_gauge_layout(source_key: torch.Tensor, source_value: torch.Tensor,
+                              key_center: torch.Tensor, value_center: torch.Tensor,
+                              key_codes: torch.Tensor, value_codes: torch.Tensor,
+                              key_scales: torch.Tensor, value_scales: torch.Tensor,
+                              exact_key_pages: torch.Tensor, exact_value_pages: torch.Tensor,
+                              request: int, layout) -> None:
+    """``prefill_page_gauge`` whose exact pages follow ``layout`` (a
+    ``page_table.ExactPageLayout``) in ``request``'s block of exact slots: the
+    kernel works the slot of each page out, so no map is built, copied or
+    checked (the check of a device map waits for the GPU)."""
+    pages, heads, key_stride, value_stride = _prefill_source_checks(
+        source_key, source_value, key_center, value_center, key_codes, value_codes, key_scales,
+        value_scales)
+    _exact_page_checks(heads, exact_key_pages, exact_value_pages)
+    _all_cuda_contiguous(exact_key_pages, exact_value_pages)
+    if request < 0:
+        raise ValueError("exact page mapping inputs must be non-negative with a tail")
+    slots = min(exact_key_pages.shape[0], exact_value_pages.shape[0])
+    _capi.call("pg_prefill_page_gauge_layout", source_key.data_ptr(), key_stride,
+               source_value.data_ptr(), value_stride, key_center.data_ptr(),
+               value_center.data_ptr(), key_codes.data_ptr(), value_codes.data_ptr(),
+               key_scales.data_ptr(), value_scales.data_ptr(), exact_key_pages.data_ptr(),
+               exact_value_pages.data_ptr(), slots, request * layout.storage, layout.prefix,
+               layout.suffix_pages.start if layout.suffix else 0, layout.suffix, layout.tail,
+               pages, heads, _stream())
