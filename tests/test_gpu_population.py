@@ -94,3 +94,29 @@ def test_layout_form_is_the_map_form(cuda, sink, suffix, initial, tail, pages, r
         assert torch.equal(_bits(a), _bits(b))
     with pytest.raises(RuntimeError, match="past the exact pages"):
         prefill_page_gauge_layout(k, v, *centers, *results[0][:4], *results[0][4:], 3, layout)
+
+
+# chunks of 64 tokens; 16 rows of the second launch; column groups that do not
+# divide the block; 4-byte rows
+@pytest.mark.parametrize("tokens,heads,pad", [(1, 1, 0), (64, 8, 0), (1025, 3, 0), (1088, 9, 0),
+                                              (65, 17, 0), (130, 3, 2), (2049, 5, 2)])
+@pytest.mark.parametrize("kind", ["plain", "tiny", "large"])
+def test_centers_are_the_exact_mean(cuda, tokens, heads, pad, kind):
+    from oracle import pg_oracle as oracle
+    from pagegauge_amd.update import token_major_centers
+
+    print(f"centers {kind} tokens={tokens} heads={heads} pad={pad}", flush=True)
+    k, v = _source(kind, tokens, heads, pad, cuda), _source(kind, tokens, heads, pad, cuda).neg()
+    if pad:
+        v = _source(kind, tokens, heads, pad, cuda)
+    for got, x in zip(token_major_centers(k, v), (k, v)):
+        want = torch.from_numpy(oracle.exact_center(x.cpu().numpy()[:, None]))
+        assert torch.equal(_bits(got.cpu()), _bits(want))
+
+
+def test_centers_of_not_finite_values_do_not_depend_on_the_width(cuda):
+    from pagegauge_amd.update import token_major_centers
+
+    results = [token_major_centers(x, x)[0] for x in
+               (_source("not_finite", 300, 2, pad, cuda) for pad in (0, 2))]
+    assert torch.equal(_bits(results[0]), _bits(results[1]))
