@@ -548,6 +548,16 @@ int32_t pg_decoder_gemv(const void* weight, int32_t n, int32_t k, const void* x,
                         int32_t swiglu, const void* residual, int64_t residual_stride, void* out,
                         int64_t out_stride, int32_t out_f32, void* stream);
 
+/* pg_decoder_gemv for batches of 1 to 16 rows, on the matrix cores at any
+ * batch (the reference decodes such batches through F.linear,
+ * scripts/benchmark_page_gauge_transformer.py:2754-2805); same arguments and
+ * roundings, any input width that is a multiple of 512; norm_weight at a
+ * width of 4096 only (elsewhere pg_rms_norm goes first). */
+int32_t pg_decoder_gemm(const void* weight, int32_t n, int32_t k, const void* x,
+                        int64_t x_stride, int32_t batch, const void* norm_weight, float eps,
+                        int32_t swiglu, const void* residual, int64_t residual_stride, void* out,
+                        int64_t out_stride, int32_t out_f32, void* stream);
+
 /* The QKV projection of a decode step fused with its cache update: the
  * decoder layer's qkv F.linear (with the input RMSNorm, as pg_decoder_gemv)
  * followed by rope_append_page_gauge_dynamic / rope_append_fp16_dynamic
@@ -575,6 +585,20 @@ int32_t pg_decoder_qkv_rope_append(const void* weight, int32_t k, const void* x,
                                    const void* value_center, int64_t center_batch_stride,
                                    int32_t pages_per_request, int32_t sink_pages,
                                    int32_t capacity_tokens, void* stream);
+
+/* pg_decoder_qkv_rope_append for batches of 1 to 16 rows and any input width
+ * that is a multiple of 512, the projection as pg_decoder_gemm (norm_weight
+ * NULL: x holds the normalised input). */
+int32_t pg_decoder_gemm_rope_append(const void* weight, int32_t k, const void* x,
+                                    int64_t x_stride, int32_t batch, const void* norm_weight,
+                                    float eps, int32_t query_heads, int32_t kv_heads,
+                                    const void* cosine, const void* sine, int64_t rope_row_stride,
+                                    int32_t rope_rows, const int32_t* positions,
+                                    int32_t position_stride, void* rotated_query, void* key_pages,
+                                    void* value_pages, const void* key_center,
+                                    const void* value_center, int64_t center_batch_stride,
+                                    int32_t pages_per_request, int32_t sink_pages,
+                                    int32_t capacity_tokens, void* stream);
 
 /* Greedy token selection of the decode loop: out[r] = argmax of row r of
  * x [rows, row_stride] float32 over its first n elements, as

@@ -114,6 +114,11 @@ PROTOTYPES = {
     "pg_decode_run_combine": (_i32, [ctypes.POINTER(DecodePlan), _p, _i64, _p, _p, _p, _p]),
     "pg_decoder_gemv": (_i32, [_p, _i32, _i32, _p, _i64, _i32, _p, _f32, _i32, _p, _i64, _p, _i64,
                                _i32, _p]),
+    "pg_decoder_gemm": (_i32, [_p, _i32, _i32, _p, _i64, _i32, _p, _f32, _i32, _p, _i64, _p, _i64,
+                               _i32, _p]),
+    "pg_decoder_gemm_rope_append": (_i32, [_p, _i32, _p, _i64, _i32, _p, _f32, _i32, _i32, _p, _p,
+                                           _i64, _i32, _p, _i32, _p, _p, _p, _p, _p, _i64, _i32,
+                                           _i32, _i32, _p]),
     "pg_decoder_qkv_rope_append": (_i32, [_p, _i32, _p, _i64, _i32, _p, _f32, _i32, _i32, _p, _p,
                                           _i64, _i32, _p, _i32, _p, _p, _p, _p, _p, _i64, _i32,
                                           _i32, _i32, _p]),

@@ -1,5 +1,5 @@
 // Decoder-step projections for gfx950: y = W x with the neighbouring
-// element-wise work fused in, for batch-1..4 decode steps.
+// element-wise work fused in, for decode steps of 1 to 16 rows.
 //
 // One launch replaces, per projection of a Mistral decoder layer
 // (scripts/benchmark_page_gauge_transformer.py:2754-2805):
@@ -18,8 +18,9 @@
 //     -- epilogue.  The completed page's INT8 finalize runs in the decode's
 //     FP16 tail pass (pg_decode_run_finalize).
 //
-// The work is HBM-bound weight streaming (M = batch <= 4): every weight byte
-// is read once.  A workgroup (4 waves; 7 for the 14336-wide down
+// The work is HBM-bound weight streaming: every weight byte is read once.
+// Batches of two rows up run on the matrix cores (decoder_matrix_kernel below);
+// one row runs on v_dot2 as follows.  A workgroup (4 waves; 7 for the 14336-wide down
 // projection, whose 4-chunk waves fit occupancy 5) owns a group of rows; the
 // 512-element chunks of a row are split over its waves (kC consecutive
 // chunks each), a
@@ -484,6 +485,321 @@ __global__ __launch_bounds__(kGemvThreads) void decoder_gemv_generic_kernel(Gemv
   }
 }
 
+// ---------------------------------------------------------------------------
+// Batches of 2 to 16 rows: the same projections on the matrix cores.
+//
+// v_mfma_f32_16x16x32_f16 with weight rows as the A operand and the (up to 16)
+// input rows as B: the whole batch costs what one row does, where v_dot2 needs
+// four instructions per 16 bytes of weights and input row, and registers for
+// every row.  A workgroup owns tiles of 16 weight rows (8 gate and 8 up rows
+// with SwiGLU; dims d..d+7 and d+64..d+71 of one head for the append), each of
+// its 8 waves an eighth of the input width; the waves' 16 x 16 sums meet in
+// LDS (two buffers, one barrier per tile).  One workgroup per CU walks the
+// tiles, and a wave keeps two tiles of its slice (32 KiB) in flight, in blocks
+// of 4 KiB that are refilled one by one, so that the stream does not stop
+// at a tile's reduction.
+//
+// The A operand wants 16 rows x 64 bytes per instruction: half cache lines.
+// Here an instruction loads 8 rows x 128 bytes instead, lanes r < 8 one step
+// of 32 elements and lanes r >= 8 the next, and each step's MFMA uses the half
+// of the operand that belongs to it: twice the MFMAs, half of every result
+// dropped, on units that idle otherwise (28672 x 4096, batch 1: 46.9 us with
+// half lines, 39.5 like this).
+//
+// kResident (width 4096): a wave's slice of the normalised input stays in
+// registers for all tiles.  Otherwise the input, normalised before the call, is
+// read again with each block of weights (from L2), and any multiple of 512 will
+// do.
+//
+// Cold weights, us for batch 2 / 4 / 16 (v_dot2 kernel for 2 / 4, hipBLASLt
+// without norm and epilogue for 16): QKV 6144 x 4096 13.8 / 13.8 / 15.9 (11.9
+// / 19.5, 17.8), output 4096 x 4096 7.8 / 8.0 / 9.8 (9.1 / 11.8, 17.6),
+// gate/up 28672 x 4096 39.3 / 39.6 / 43.2 (40.5 / 53.7, 60), down 4096 x 14336
+// 20.3 / 21.3 / 28.3 (28.7 / 38.2, 25.7), head 32768 x 4096 44.0 / 44.3 / 46.2
+// (42.7 / 56.2, 58.7).
+// ---------------------------------------------------------------------------
+typedef float v4f_t __attribute__((ext_vector_type(4)));
+constexpr int kTileRows = 16;
+constexpr int kMatrixBatch = 16;
+constexpr int kMatrixWaves = 8;
+constexpr int kMatrixStep = 32;      // input elements per MFMA
+constexpr int kSteps = 4;            // steps per block of loads
+constexpr int kResidentBlocks = 4;   // blocks of a resident slice
+constexpr int kResidentWidth = kMatrixWaves * kMatrixStep * kSteps * kResidentBlocks;   // 4096
+constexpr int kStreamRing = 2;       // blocks in flight with a streamed input
+
+// Sums over the rows' four lanes (16 apart).
+__device__ __forceinline__ float group4_sum(float v) {
+  v += __shfl_xor(v, 16, kWave);
+  v += __shfl_xor(v, 32, kWave);
+  return v;
+}
+
+// Orders LDS accesses across the workgroup's barrier; loads stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <bool kSwiglu, bool kRope, bool kResident>
+__global__ __launch_bounds__(kWave * kMatrixWaves, kMatrixWaves / 4) void decoder_matrix_kernel(
+    GemvArgs a, int batch, int tiles) {
+  constexpr bool kPaired = kSwiglu || kRope;      // two weight rows make one output (pair)
+  constexpr int kOutRows = kPaired ? kTileRows / 2 : kTileRows;
+  constexpr int kRing = kResident ? kResidentBlocks : kStreamRing;   // blocks in flight
+  __shared__ __attribute__((aligned(16))) float partial[2][kMatrixWaves][kTileRows * kMatrixBatch];
+  __shared__ float squares[kMatrixWaves][kMatrixBatch];
+  __shared__ __attribute__((aligned(16))) uint16_t norm_lds[kResident ? kResidentWidth : 8];
+  const int wave = threadIdx.x / kWave;
+  const int lane = threadIdx.x % kWave;
+  const int r = lane & 15;             // weight row of the tile (A), input row (B)
+  const int g = lane >> 4;
+  const int steps = kResident ? kResidentBlocks * kSteps : a.k / (kMatrixWaves * kMatrixStep);   // per wave
+  const int blocks = kResident ? kRing : (steps + kSteps - 1) / kSteps;                // per tile
+  const int slice = wave * steps * kMatrixStep + 8 * g;
+  const int mine = (tiles - static_cast<int>(blockIdx.x) + static_cast<int>(gridDim.x) - 1) /
+                   static_cast<int>(gridDim.x);
+  const uint16_t* x = a.x + min(r, batch - 1) * a.x_stride + slice;
+
+  // Block ``block`` (of kSteps steps) of this workgroup's ``count``-th tile.
+  // Register w[s + h] (s even) holds half h of the tile (8 weight rows) for
+  // steps s and s + 1: lanes r < 8 the first, r >= 8 the second, so that an
+  // instruction reads 128 contiguous bytes of each row.
+  auto load = [&](int count, int block, v4u_t (&w)[kSteps]) {
+    const int tile = blockIdx.x + count * gridDim.x;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      int first, rows;                 // first weight row, rows of this half that exist
+      if constexpr (kRope) {
+        first = (tile / 8) * kHeadDim + (tile % 8) * 8 + 64 * h;
+        rows = 8;
+      } else if constexpr (kSwiglu) {
+        first = tile * 8 + h * a.out_rows;
+        rows = a.out_rows - tile * 8;
+      } else {
+        first = min(tile * kTileRows + 8 * h, a.out_rows - 1);
+        rows = a.out_rows - first;
+      }
+      const uint16_t* at = a.weight + static_cast<int64_t>(first) * a.k + min(r & 7, rows - 1) * a.k + slice;
+#pragma unroll
+      for (int s = 0; s < kSteps; s += 2) {
+        // a step past the slice re-reads its last one; no product uses it
+        const int step = kResident ? block * kSteps + s + (r >> 3)
+                                   : min(block * kSteps + s + (r >> 3), steps - 1);
+        w[s + h] = __builtin_nontemporal_load(reinterpret_cast<const v4u_t*>(at + step * kMatrixStep));
+      }
+    }
+  };
+  auto load_x = [&](int block, v4u_t (&xv)[kSteps]) {
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+      const int step = kResident ? block * kSteps + s : min(block * kSteps + s, steps - 1);
+      xv[s] = *reinterpret_cast<const v4u_t*>(x + step * kMatrixStep);
+    }
+  };
+
+  v4u_t w[kRing][kSteps], xv[kRing][kSteps];
+  const bool norm = a.norm_weight != nullptr;      // resident only
+  // resident: thread t brings the norm weights 8t..8t+7 to LDS
+  v4u_t norm_part = {0u, 0u, 0u, 0u};
+  if (kResident && norm) norm_part = *reinterpret_cast<const v4u_t*>(a.norm_weight + 8 * threadIdx.x);
+  int next_count = 0, next_block = 0;  // the next block to request
+  auto advance = [&]() {
+    if (++next_block == blocks) {
+      next_block = 0;
+      ++next_count;
+    }
+  };
+#pragma unroll
+  for (int b = 0; b < kRing; ++b) {
+    if constexpr (kResident) {
+      load(0, b, w[b]);
+      load_x(b, xv[b]);
+      __builtin_amdgcn_sched_barrier(0);
+    } else if (next_count < mine) {
+      load(next_count, next_block, w[b]);
+      load_x(next_block, xv[b]);
+      advance();
+    }
+  }
+  if constexpr (kResident) {
+    if (norm) {
+      float ss = 0.0f;
+#pragma unroll
+      for (int b = 0; b < kRing; ++b)
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s) ss += squares8(xv[b][s]);
+      *reinterpret_cast<v4u_t*>(&norm_lds[8 * threadIdx.x]) = norm_part;
+      ss = group4_sum(ss);
+      if (g == 0) squares[wave][r] = ss;
+      lds_barrier();
+      float total = 0.0f;
+#pragma unroll
+      for (int i = 0; i < kMatrixWaves; ++i) total += squares[i][r];
+      const float inv = rsqrtf(total / static_cast<float>(a.k) + a.eps);
+#pragma unroll
+      for (int b = 0; b < kRing; ++b) {
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s) {
+          // opaque: the float32 values of the squares are not kept for this
+          // (they would not fit the registers)
+          v4u_t raw = xv[b][s];
+          asm volatile("" : "+v"(raw));
+          xv[b][s] = normalize8(raw, *reinterpret_cast<const v4u_t*>(
+                                         &norm_lds[slice + (b * kSteps + s) * kMatrixStep]), inv);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+
+  // acc[h][j]: half h of the tile with steps of parity j.  Its valid rows are
+  // those whose lanes held that step: C rows 8j..8j+7.
+  v4f_t acc[2][2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[h][j] = v4f_t{0.0f, 0.0f, 0.0f, 0.0f};
+  AppendInputs append_in{};
+  auto compute = [&](int count, int block, v4u_t (&wb)[kSteps], v4u_t (&xb)[kSteps]) {
+    const int tile = blockIdx.x + count * gridDim.x;
+    if constexpr (kRope) {
+      // the row pairs' RoPE / center inputs, requested before the products
+      if (block == 0 && static_cast<int>(threadIdx.x) / 8 < batch)
+        append_in = append_inputs(a, threadIdx.x / 8, tile * 8 + threadIdx.x % 8);
+    }
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+      if (!kResident && block * kSteps + s >= steps) break;
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        acc[h][s & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+            __builtin_bit_cast(v8h_t, wb[(s & ~1) + h]), __builtin_bit_cast(v8h_t, xb[s]),
+            acc[h][s & 1], 0, 0, 0);
+    }
+    if (block != blocks - 1) return;
+    // lane (input row r): rows 4 (g % 2).. of half h, the even steps' sum where
+    // g < 2 and the odd steps' where g >= 2; the two are added, and lanes g
+    // keep rows 4g..4g+3 of the tile
+    v4f_t sum[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const v4f_t own = g < 2 ? acc[h][0] : acc[h][1];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum[h][e] = own[e] + __shfl_xor(own[e], 32, kWave);
+      acc[h][0] = acc[h][1] = v4f_t{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    float (&sums)[kMatrixWaves][kTileRows * kMatrixBatch] = partial[count & 1];
+    *reinterpret_cast<v4f_t*>(&sums[wave][r * kTileRows + 4 * g]) = g < 2 ? sum[0] : sum[1];
+    lds_barrier();
+    // a thread per output: input row b, output row o of the tile
+    const int b = threadIdx.x / kOutRows;
+    const int o = threadIdx.x % kOutRows;
+    if (b >= batch) return;
+    float y0 = 0.0f, y1 = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kMatrixWaves; ++i) {
+      y0 += sums[i][b * kTileRows + o];
+      if (kPaired) y1 += sums[i][b * kTileRows + 8 + o];
+    }
+    if constexpr (kRope) {
+      append_pair(a, b, tile * 8 + o, y0, y1, append_in);
+    } else {
+      const int row = tile * kOutRows + o;
+      if (row < a.out_rows) store_output(a, b, row, y0, y1);
+    }
+  };
+  if constexpr (kResident) {
+    // two tiles in turn, a block's registers refilled two tiles ahead as soon
+    // as its products are done
+    v4u_t w2[kRing][kSteps];
+    if (mine > 1) {
+#pragma unroll
+      for (int b = 0; b < kRing; ++b) {
+        load(1, b, w2[b]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    for (int count = 0; count < mine; count += 2) {
+#pragma unroll
+      for (int b = 0; b < kRing; ++b) {
+        compute(count, b, w[b], xv[b]);
+        __builtin_amdgcn_sched_barrier(0);   // the next loads take the registers just freed
+        if (count + 2 < mine) load(count + 2, b, w[b]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (count + 1 >= mine) break;
+#pragma unroll
+      for (int b = 0; b < kRing; ++b) {
+        compute(count + 1, b, w2[b], xv[b]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (count + 3 < mine) load(count + 3, b, w2[b]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  } else {
+    int count = 0, block = 0;
+    while (count < mine) {
+#pragma unroll
+      for (int b = 0; b < kRing; ++b) {
+        if (count >= mine) break;
+        compute(count, block, w[b], xv[b]);
+        if (++block == blocks) {
+          block = 0;
+          ++count;
+        }
+        if (next_count < mine) {
+          load(next_count, next_block, w[b]);
+          load_x(next_block, xv[b]);
+          advance();
+        }
+      }
+    }
+  }
+}
+
+constexpr int kMatrixBlocks = 256;   // one 16-wave workgroup per CU
+
+// Batches the matrix kernel takes; a.swiglu / ``rope`` pick the epilogue.
+template <bool kRope>
+int32_t launch_matrix(const GemvArgs& a, int batch, hipStream_t s, const char* what) {
+  const int per_tile = a.swiglu || kRope ? kTileRows / 2 : kTileRows;
+  const int rows = kRope ? a.out_rows / 2 : a.out_rows;
+  const int tiles = (rows + per_tile - 1) / per_tile;
+  const dim3 grid(static_cast<unsigned>(tiles < kMatrixBlocks ? tiles : kMatrixBlocks));
+  const auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(kWave * kMatrixWaves), 0, s, a, batch, tiles);
+  };
+  const bool resident = a.k == kResidentWidth;
+  if constexpr (kRope) {
+    if (resident) launch(decoder_matrix_kernel<false, true, true>);
+    else launch(decoder_matrix_kernel<false, true, false>);
+  } else if (a.swiglu) {
+    if (resident) launch(decoder_matrix_kernel<true, false, true>);
+    else launch(decoder_matrix_kernel<true, false, false>);
+  } else {
+    if (resident) launch(decoder_matrix_kernel<false, false, true>);
+    else launch(decoder_matrix_kernel<false, false, false>);
+  }
+  return check_launch(what);
+}
+
+// Whether a batch of 1 to 4 rows runs on the matrix cores: at the widths with
+// kernels of their own, from 3 rows on, and with 2 rows except behind a norm
+// without SwiGLU (QKV, head), where the v_dot2 kernel is the faster one (figures
+// above).  At other widths the staged kernel stays ahead up to 4 rows (us for 2
+// / 4 rows, staged against streamed: 5120 x 5120 12.2 / 14.4 against 15.7 /
+// 16.8, 2048 x 5632 8.1 / 10.4 against 9.3 / 10.0).  The rule looks at nothing
+// but the projection, so that the QKV projection with and without the cache
+// update gives the same bits.
+bool matrix_batch(const GemvArgs& a, int batch) {
+  const bool own_width = a.k == kResidentWidth || (a.k == 14336 && !a.swiglu && !a.norm_weight);
+  if (!own_width || batch < 2) return false;
+  return batch > 2 || a.k != kResidentWidth || a.norm_weight == nullptr || a.swiglu;
+}
+
+// The v_dot2 kernels.
 template <int kBatch>
 int32_t launch_gemv(GemvArgs a, hipStream_t s) {
   const int chunks = a.k / kChunk;
@@ -493,32 +809,40 @@ int32_t launch_gemv(GemvArgs a, hipStream_t s) {
     blocks = (blocks + a.iterations - 1) / a.iterations;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(kWave * waves), 0, s, a);
   };
-  if (chunks == 8 && !a.swiglu) {                 // k = 4096
-    if (a.out_rows > 8192)
-      blocked(decoder_gemv_kernel<kBatch, PG_GEMV_ROWS_4096_LARGE, 2, false>, PG_GEMV_ROWS_4096_LARGE);
-    else
-      blocked(decoder_gemv_kernel<kBatch, PG_GEMV_ROWS_4096, 2, false>, PG_GEMV_ROWS_4096);
-  } else if (chunks == 8) {
-    blocked(decoder_gemv_kernel<kBatch, PG_GEMV_ROWS_4096, 2, true>, PG_GEMV_ROWS_4096);
-  } else if (chunks == 28 && !a.swiglu) {         // k = 14336
+  if constexpr (kBatch <= 2) {
+    if (chunks == 8 && !a.swiglu) {                 // k = 4096
+      if (a.out_rows > 8192)
+        blocked(decoder_gemv_kernel<kBatch, PG_GEMV_ROWS_4096_LARGE, 2, false>, PG_GEMV_ROWS_4096_LARGE);
+      else
+        blocked(decoder_gemv_kernel<kBatch, PG_GEMV_ROWS_4096, 2, false>, PG_GEMV_ROWS_4096);
+      return check_launch("decoder_gemv");
+    }
+  }
+  if constexpr (kBatch == 1) {
+    if (chunks == 8) {
+      blocked(decoder_gemv_kernel<1, PG_GEMV_ROWS_4096, 2, true>, PG_GEMV_ROWS_4096);
+      return check_launch("decoder_gemv");
+    }
+  }
+  if (chunks == 28 && !a.swiglu && (kBatch == 1 || a.norm_weight)) {   // k = 14336
     static_assert(28 % PG_GEMV_WAVES_14336 == 0, "k = 14336 splits into whole chunks per wave");
     constexpr int kWaves14336 = PG_GEMV_WAVES_14336;
     blocked(decoder_gemv_kernel<kBatch, PG_GEMV_ROWS_14336, 28 / kWaves14336, false, false,
                                 kWaves14336>,
             PG_GEMV_ROWS_14336, kWaves14336);
-  } else {
-    const size_t lds = static_cast<size_t>(kBatch) * a.k * sizeof(uint16_t);
-    if (lds > kMaxStagedBytes)
-      return fail(PG_ERROR_UNSUPPORTED, "batch * input width exceeds the 32768-element LDS staging");
-    const int per_wave = a.swiglu ? 1 : 2;
-    const int64_t waves = (static_cast<int64_t>(a.out_rows) + per_wave - 1) / per_wave;
-    int64_t blocks = (waves + kGemvWaves - 1) / kGemvWaves;
-    a.iterations = static_cast<int>((blocks + kMaxBlocks - 1) / kMaxBlocks);
-    blocks = (waves + static_cast<int64_t>(kGemvWaves) * a.iterations - 1) /
-             (static_cast<int64_t>(kGemvWaves) * a.iterations);
-    hipLaunchKernelGGL(decoder_gemv_generic_kernel<kBatch>, dim3(static_cast<unsigned>(blocks)),
-                       dim3(kGemvThreads), lds, s, a);
+    return check_launch("decoder_gemv");
   }
+  const size_t lds = static_cast<size_t>(kBatch) * a.k * sizeof(uint16_t);
+  if (lds > kMaxStagedBytes)
+    return fail(PG_ERROR_UNSUPPORTED, "batch * input width exceeds the 32768-element LDS staging");
+  const int per_wave = a.swiglu ? 1 : 2;
+  const int64_t waves = (static_cast<int64_t>(a.out_rows) + per_wave - 1) / per_wave;
+  int64_t blocks = (waves + kGemvWaves - 1) / kGemvWaves;
+  a.iterations = static_cast<int>((blocks + kMaxBlocks - 1) / kMaxBlocks);
+  blocks = (waves + static_cast<int64_t>(kGemvWaves) * a.iterations - 1) /
+           (static_cast<int64_t>(kGemvWaves) * a.iterations);
+  hipLaunchKernelGGL(decoder_gemv_generic_kernel<kBatch>, dim3(static_cast<unsigned>(blocks)),
+                     dim3(kGemvThreads), lds, s, a);
   return check_launch("decoder_gemv");
 }
 
@@ -606,25 +930,26 @@ int32_t launch_qkv_append(GemvArgs a, hipStream_t s) {
 
 using namespace pg;
 
-extern "C" int32_t pg_decoder_gemv(const void* weight, int32_t n, int32_t k, const void* x,
-                                   int64_t x_stride, int32_t batch, const void* norm_weight,
-                                   float eps, int32_t swiglu, const void* residual,
-                                   int64_t residual_stride, void* out, int64_t out_stride,
-                                   int32_t out_f32, void* stream) {
-  clear_error();
+namespace {
+
+// Checks shared by both projection entry points; ``most``: their largest batch.
+int32_t projection_args(const void* weight, int32_t n, int32_t k, const void* x, int64_t x_stride,
+                        int32_t batch, int32_t most, const void* norm_weight, float eps,
+                        int32_t swiglu, const void* residual, int64_t residual_stride, void* out,
+                        int64_t out_stride, int32_t out_f32, GemvArgs& a) {
   if (weight == nullptr || x == nullptr || out == nullptr)
     return fail(PG_ERROR_INVALID_ARGUMENT, "null tensor pointer");
   if (n <= 0 || k <= 0 || k % kChunk)
     return fail(PG_ERROR_INVALID_ARGUMENT, "rows must be positive and the input width a multiple of 512");
-  if (batch < 1 || batch > kMaxBatch)
-    return fail(PG_ERROR_UNSUPPORTED, "decoder projections take a batch of 1 to 4 rows");
+  if (batch < 1 || batch > most)
+    return fail(PG_ERROR_UNSUPPORTED,
+                "decoder projections take a batch of 1 to " + std::to_string(most) + " rows");
   if (swiglu && n % 2)
     return fail(PG_ERROR_INVALID_ARGUMENT, "a SwiGLU projection needs gate and up rows (even n)");
   const int out_rows = swiglu ? n / 2 : n;
   if (x_stride < k || x_stride % 8 || (residual != nullptr && residual_stride < out_rows) ||
       out_stride < out_rows)
     return fail(PG_ERROR_INVALID_ARGUMENT, "row strides must cover the rows (input stride a multiple of 8)");
-  GemvArgs a{};
   a.weight = static_cast<const uint16_t*>(weight);
   a.x = static_cast<const uint16_t*>(x);
   a.x_stride = x_stride;
@@ -639,33 +964,38 @@ extern "C" int32_t pg_decoder_gemv(const void* weight, int32_t n, int32_t k, con
   a.n = n;
   a.out_rows = out_rows;
   a.k = k;
-  hipStream_t s = as_stream(stream);
-  switch (batch) {
-    case 1: return launch_gemv<1>(a, s);
-    case 2: return launch_gemv<2>(a, s);
-    case 3: return launch_gemv<3>(a, s);
-    default: return launch_gemv<4>(a, s);
-  }
+  return PG_OK;
 }
 
-extern "C" int32_t pg_decoder_qkv_rope_append(
-    const void* weight, int32_t k, const void* x, int64_t x_stride, int32_t batch,
-    const void* norm_weight, float eps, int32_t query_heads, int32_t kv_heads, const void* cosine,
-    const void* sine, int64_t rope_row_stride, int32_t rope_rows, const int32_t* positions,
-    int32_t position_stride, void* rotated_query, void* key_pages, void* value_pages,
-    const void* key_center, const void* value_center, int64_t center_batch_stride,
-    int32_t pages_per_request, int32_t sink_pages, int32_t capacity_tokens, void* stream) {
-  clear_error();
+// The matrix kernel applies a norm where it keeps the input.
+int32_t norm_width(const GemvArgs& a) {
+  if (a.norm_weight != nullptr && a.k != kResidentWidth)
+    return fail(PG_ERROR_UNSUPPORTED, "the norm of a batched projection takes a 4096-wide input");
+  return PG_OK;
+}
+
+// Checks shared by both QKV append entry points.
+int32_t append_args(const void* weight, int32_t k, const void* x, int64_t x_stride, int32_t batch,
+                    int32_t most, const void* norm_weight, float eps, int32_t query_heads,
+                    int32_t kv_heads, const void* cosine, const void* sine,
+                    int64_t rope_row_stride, int32_t rope_rows, const int32_t* positions,
+                    int32_t position_stride, void* rotated_query, void* key_pages,
+                    void* value_pages, const void* key_center, const void* value_center,
+                    int64_t center_batch_stride, int32_t pages_per_request, int32_t sink_pages,
+                    int32_t capacity_tokens, GemvArgs& a) {
   if (weight == nullptr || x == nullptr || cosine == nullptr || sine == nullptr ||
       positions == nullptr || rotated_query == nullptr || key_pages == nullptr ||
       value_pages == nullptr)
     return fail(PG_ERROR_INVALID_ARGUMENT, "null tensor pointer");
   if ((key_center == nullptr) != (value_center == nullptr))
     return fail(PG_ERROR_INVALID_ARGUMENT, "key and value centers go together");
-  if (k != 8 * kChunk)
+  if (most <= kMaxBatch && k != kResidentWidth)
     return fail(PG_ERROR_UNSUPPORTED, "the QKV append projection takes a 4096-wide input");
-  if (batch < 1 || batch > kMaxBatch)
-    return fail(PG_ERROR_UNSUPPORTED, "decoder projections take a batch of 1 to 4 rows");
+  if (k <= 0 || k % kChunk)
+    return fail(PG_ERROR_INVALID_ARGUMENT, "the input width must be a multiple of 512");
+  if (batch < 1 || batch > most)
+    return fail(PG_ERROR_UNSUPPORTED,
+                "decoder projections take a batch of 1 to " + std::to_string(most) + " rows");
   if (query_heads <= 0 || kv_heads <= 0 || query_heads % kv_heads)
     return fail(PG_ERROR_INVALID_ARGUMENT, "query heads must be a positive multiple of KV heads");
   if (x_stride < k || x_stride % 8 || rope_row_stride < kHeadDim || rope_rows <= 0 ||
@@ -678,7 +1008,6 @@ extern "C" int32_t pg_decoder_qkv_rope_append(
   if (key_center != nullptr && center_batch_stride < static_cast<int64_t>(kv_heads) * kHeadDim &&
       batch > 1)
     return fail(PG_ERROR_INVALID_ARGUMENT, "center batch stride must cover the KV heads");
-  GemvArgs a{};
   a.weight = static_cast<const uint16_t*>(weight);
   a.x = static_cast<const uint16_t*>(x);
   a.x_stride = x_stride;
@@ -705,13 +1034,83 @@ extern "C" int32_t pg_decoder_qkv_rope_append(
   p.pages_per_request = pages_per_request;
   p.sink_pages = sink_pages;
   p.capacity_tokens = capacity_tokens;
+  return PG_OK;
+}
+
+}  // namespace
+
+extern "C" int32_t pg_decoder_gemv(const void* weight, int32_t n, int32_t k, const void* x,
+                                   int64_t x_stride, int32_t batch, const void* norm_weight,
+                                   float eps, int32_t swiglu, const void* residual,
+                                   int64_t residual_stride, void* out, int64_t out_stride,
+                                   int32_t out_f32, void* stream) {
+  clear_error();
+  GemvArgs a{};
+  if (int32_t rc = projection_args(weight, n, k, x, x_stride, batch, kMaxBatch, norm_weight, eps,
+                                   swiglu, residual, residual_stride, out, out_stride, out_f32, a))
+    return rc;
   hipStream_t s = as_stream(stream);
+  if (matrix_batch(a, batch)) return launch_matrix<false>(a, batch, s, "decoder_gemv");
   switch (batch) {
-    case 1: return launch_qkv_append<1>(a, s);
-    case 2: return launch_qkv_append<2>(a, s);
-    case 3: return launch_qkv_append<3>(a, s);
-    default: return launch_qkv_append<4>(a, s);
+    case 1: return launch_gemv<1>(a, s);
+    case 2: return launch_gemv<2>(a, s);
+    case 3: return launch_gemv<3>(a, s);
+    default: return launch_gemv<4>(a, s);
   }
+}
+
+extern "C" int32_t pg_decoder_gemm(const void* weight, int32_t n, int32_t k, const void* x,
+                                   int64_t x_stride, int32_t batch, const void* norm_weight,
+                                   float eps, int32_t swiglu, const void* residual,
+                                   int64_t residual_stride, void* out, int64_t out_stride,
+                                   int32_t out_f32, void* stream) {
+  clear_error();
+  GemvArgs a{};
+  if (int32_t rc = projection_args(weight, n, k, x, x_stride, batch, kMatrixBatch, norm_weight,
+                                   eps, swiglu, residual, residual_stride, out, out_stride,
+                                   out_f32, a))
+    return rc;
+  if (int32_t rc = norm_width(a)) return rc;
+  return launch_matrix<false>(a, batch, as_stream(stream), "decoder_gemm");
+}
+
+extern "C" int32_t pg_decoder_qkv_rope_append(
+    const void* weight, int32_t k, const void* x, int64_t x_stride, int32_t batch,
+    const void* norm_weight, float eps, int32_t query_heads, int32_t kv_heads, const void* cosine,
+    const void* sine, int64_t rope_row_stride, int32_t rope_rows, const int32_t* positions,
+    int32_t position_stride, void* rotated_query, void* key_pages, void* value_pages,
+    const void* key_center, const void* value_center, int64_t center_batch_stride,
+    int32_t pages_per_request, int32_t sink_pages, int32_t capacity_tokens, void* stream) {
+  clear_error();
+  GemvArgs a{};
+  if (int32_t rc = append_args(weight, k, x, x_stride, batch, kMaxBatch, norm_weight, eps,
+                               query_heads, kv_heads, cosine, sine, rope_row_stride, rope_rows,
+                               positions, position_stride, rotated_query, key_pages, value_pages,
+                               key_center, value_center, center_batch_stride, pages_per_request,
+                               sink_pages, capacity_tokens, a))
+    return rc;
+  hipStream_t s = as_stream(stream);
+  if (matrix_batch(a, batch)) return launch_matrix<true>(a, batch, s, "decoder_qkv_rope_append");
+  return batch == 1 ? launch_qkv_append<1>(a, s) : launch_qkv_append<2>(a, s);
+}
+
+extern "C" int32_t pg_decoder_gemm_rope_append(
+    const void* weight, int32_t k, const void* x, int64_t x_stride, int32_t batch,
+    const void* norm_weight, float eps, int32_t query_heads, int32_t kv_heads, const void* cosine,
+    const void* sine, int64_t rope_row_stride, int32_t rope_rows, const int32_t* positions,
+    int32_t position_stride, void* rotated_query, void* key_pages, void* value_pages,
+    const void* key_center, const void* value_center, int64_t center_batch_stride,
+    int32_t pages_per_request, int32_t sink_pages, int32_t capacity_tokens, void* stream) {
+  clear_error();
+  GemvArgs a{};
+  if (int32_t rc = append_args(weight, k, x, x_stride, batch, kMatrixBatch, norm_weight, eps,
+                               query_heads, kv_heads, cosine, sine, rope_row_stride, rope_rows,
+                               positions, position_stride, rotated_query, key_pages, value_pages,
+                               key_center, value_center, center_batch_stride, pages_per_request,
+                               sink_pages, capacity_tokens, a))
+    return rc;
+  if (int32_t rc = norm_width(a)) return rc;
+  return launch_matrix<true>(a, batch, as_stream(stream), "decoder_gemm_rope_append");
 }
 
 extern "C" int32_t pg_argmax_f32(const float* x, int32_t rows, int32_t n, int64_t row_stride,

@@ -127,6 +127,14 @@ def projection(weight: torch.Tensor, x: torch.Tensor, out: torch.Tensor, *,
     weight rows are [gate; up] and ``out[i] = silu(gate_i) * up_i`` (FP16
     ops, ``out`` has N/2 columns); then ``residual`` added in FP16
     (``residual`` may be ``out``).  ``out`` is FP16 or float32 [B, N']."""
+    return _projection("pg_decoder_gemv", weight, x, out, norm_weight, eps, swiglu, residual)
+
+
+def _projection(entry: str, weight: torch.Tensor, x: torch.Tensor, out: torch.Tensor,
+                norm_weight: Optional[torch.Tensor], eps: float, swiglu: bool,
+                residual: Optional[torch.Tensor]) -> torch.Tensor:
+    """``projection`` through ``entry``: ``pg_decoder_gemv`` (up to 4 rows) or
+    ``pg_decoder_gemm`` (up to 16)."""
     from . import _capi
 
     n, k = int(weight.shape[0]), int(weight.shape[1])
@@ -146,7 +154,7 @@ def projection(weight: torch.Tensor, x: torch.Tensor, out: torch.Tensor, *,
     out_f32 = out.dtype == torch.float32
     if not out_f32 and out.dtype != torch.float16:
         raise ValueError("projection output must be FP16 or float32")
-    _capi.call("pg_decoder_gemv", weight.data_ptr(), n, k, x.data_ptr(), x.stride(0), batch,
+    _capi.call(entry, weight.data_ptr(), n, k, x.data_ptr(), x.stride(0), batch,
                None if norm_weight is None else norm_weight.data_ptr(), float(eps), int(swiglu),
                None if residual is None else residual.data_ptr(),
                0 if residual is None else residual.stride(0), out.data_ptr(), out.stride(0),
@@ -167,6 +175,16 @@ def qkv_rope_append(weight: torch.Tensor, x: torch.Tensor, *, norm_weight: torch
     ``projection`` followed by ``rope_append_page_gauge_dynamic`` /
     ``rope_append_fp16_dynamic``, except that the PageGauge page finalize is
     left to the decode (``finalize=`` of its run)."""
+    _qkv_rope_append("pg_decoder_qkv_rope_append", weight, x, norm_weight, eps, query_heads,
+                     kv_heads, cos, sin, positions, rotated_query, key_pages, value_pages,
+                     key_center, value_center, pages_per_request, sink_pages, capacity_tokens)
+
+
+def _qkv_rope_append(entry: str, weight, x, norm_weight, eps, query_heads, kv_heads, cos, sin,
+                     positions, rotated_query, key_pages, value_pages, key_center, value_center,
+                     pages_per_request, sink_pages, capacity_tokens) -> None:
+    """``qkv_rope_append`` through ``entry`` (``pg_decoder_gemm_rope_append``
+    takes up to 16 rows; without ``norm_weight``, ``x`` is normalised)."""
     from . import _capi
 
     batch, k = int(x.shape[0]), int(x.shape[1])
@@ -182,10 +200,11 @@ def qkv_rope_append(weight: torch.Tensor, x: torch.Tensor, *, norm_weight: torch
             raise ValueError(f"{name} must be contiguous FP16")
     if positions.dtype != torch.int32 or positions.numel() not in (1, batch):
         raise ValueError("positions must be int32, one shared or one per row")
-    tensors = (weight, x, norm_weight, cos, sin, positions, rotated_query, key_pages, value_pages)
+    tensors = (weight, x, cos, sin, positions, rotated_query, key_pages, value_pages,
+               *(() if norm_weight is None else (norm_weight,)))
     if not all(t.is_cuda and t.device == weight.device for t in tensors):
         raise ValueError("all tensors must be on the weights' CUDA device")
-    if norm_weight.dtype != torch.float16 or norm_weight.numel() != k:
+    if norm_weight is not None and (norm_weight.dtype != torch.float16 or norm_weight.numel() != k):
         raise ValueError("norm weight must be FP16 [K]")
     if cos.shape != sin.shape or cos.dim() != 2 or cos.shape[1] != DIM:
         raise ValueError("RoPE tables must be matching [positions, 128] tensors")
@@ -208,8 +227,8 @@ def qkv_rope_append(weight: torch.Tensor, x: torch.Tensor, *, norm_weight: torch
             raise ValueError("the exact ring needs at least one tail page after the sink")
     stride = 1 if positions.numel() == batch and batch > 1 else 0
     center_stride = 0 if key_center is None else kv_heads * DIM
-    _capi.call("pg_decoder_qkv_rope_append", weight.data_ptr(), k, x.data_ptr(), x.stride(0),
-               batch, norm_weight.data_ptr(), float(eps), query_heads, kv_heads, cos.data_ptr(),
+    _capi.call(entry, weight.data_ptr(), k, x.data_ptr(), x.stride(0),
+               batch, None if norm_weight is None else norm_weight.data_ptr(), float(eps), query_heads, kv_heads, cos.data_ptr(),
                sin.data_ptr(), cos.stride(0), int(cos.shape[0]), positions.data_ptr(), stride,
                rotated_query.data_ptr(), key_pages.data_ptr(), value_pages.data_ptr(),
                None if key_center is None else key_center.data_ptr(),
@@ -744,11 +763,39 @@ class PageGaugeDecoder:
         self.fused_append = append_ok if fused_append is None else fused_append
         if self.fused_append and not append_ok:
             raise ValueError("the fused cache update needs fused projections and hidden 4096")
+        # larger batches: the same steps through the matrix-core projections,
+        # where the weights are laid out as they read them; otherwise (and with
+        # ``fused=False``) torch operators
+        self.batched = (fused is None and not ok and self._matrix_projections_take(weights,
+                                                                                    batch_size))
+        self._append_in_projection = self.fused_append or (self.batched and fused_append is None)
+        self._projection_entry = "pg_decoder_gemm" if self.batched else "pg_decoder_gemv"
+        self._append_entry = ("pg_decoder_gemm_rope_append" if self.batched
+                              else "pg_decoder_qkv_rope_append")
         self._hidden = torch.empty(batch_size, cfg.hidden, device=device, dtype=torch.float16)
         self._qkv = torch.empty(batch_size, cfg.qkv_width, device=device, dtype=torch.float16)
         self._activation = torch.empty(batch_size, cfg.intermediate, device=device,
                                        dtype=torch.float16)
         self._logits = torch.empty(batch_size, cfg.vocab, device=device, dtype=torch.float32)
+
+    @staticmethod
+    def _matrix_projections_take(weights: DecoderWeights, batch_size: int) -> bool:
+        """``pg_decoder_gemm`` takes up to 16 rows, widths that are multiples
+        of 512 (up to 16384 for the norm) and contiguous 16-byte aligned FP16
+        weights.  At widths other than 4096 every tile of weights re-reads the
+        input, which torch operators overtake as batch x width grows (four
+        layers and head, batch 16: 5120 wide 850 us against 1158 in torch
+        operators, 8192 wide 1839 against 1755; batch 8, 8192 wide 1513
+        against 1714)."""
+        cfg = weights.config
+        if cfg.hidden != 4096 and batch_size * cfg.hidden > 98304:
+            return False
+        tensors = [weights.embed, weights.norm, weights.lm_head,
+                   *(t for layer in weights.layers for t in layer.values())]
+        return (batch_size <= 16 and cfg.hidden % 512 == 0 and cfg.hidden <= 16384
+                and cfg.intermediate % 512 == 0
+                and _on_current_device(*tensors)
+                and all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in tensors))
 
     # -- plan --------------------------------------------------------------
     def plan(self, context: int) -> None:
@@ -859,26 +906,35 @@ class PageGaugeDecoder:
             c.exact_value[layer], c.key_codes[layer], c.value_codes[layer], c.key_scales[layer],
             c.value_scales[layer], self.exact_fixed_pages)
 
+    def _norm_input(self, weight: torch.Tensor):
+        """(input, norm weight) of a projection of the normed hidden state:
+        the batched projections apply the norm themselves at a width of 4096
+        and take it applied elsewhere."""
+        if self.batched and self.config.hidden != 4096:
+            return _norm_rows(self._hidden, weight, self.config.rms_eps, None), None
+        return self._hidden, weight
+
     def _qkv_append(self, layer: int) -> None:
         """QKV projection + RoPE + cache append in one launch."""
         cfg = self.config
         w = self.weights.layers[layer]
         c = self.cache
-        common = dict(norm_weight=w["input_norm"], eps=cfg.rms_eps, query_heads=cfg.q_heads,
+        x, norm = self._norm_input(w["input_norm"])
+        common = dict(norm_weight=norm, eps=cfg.rms_eps, query_heads=cfg.q_heads,
                       kv_heads=cfg.kv_heads, cos=self.rope_cos, sin=self.rope_sin,
                       positions=self.device_position, rotated_query=self.rotated_query)
         if self.backend == "fp16":
-            qkv_rope_append(w["qkv"], self._hidden, key_pages=c.key[layer],
-                            value_pages=c.value[layer], key_center=None, value_center=None,
-                            pages_per_request=c.pages_per_request, sink_pages=0,
-                            capacity_tokens=c.pages_per_request * PAGE, **common)
+            _qkv_rope_append(self._append_entry, w["qkv"], x, key_pages=c.key[layer],
+                             value_pages=c.value[layer], key_center=None, value_center=None,
+                             pages_per_request=c.pages_per_request, sink_pages=0,
+                             capacity_tokens=c.pages_per_request * PAGE, **common)
             return
-        qkv_rope_append(w["qkv"], self._hidden, key_pages=c.exact_key[layer],
-                        value_pages=c.exact_value[layer], key_center=c.key_center[layer],
-                        value_center=c.value_center[layer],
-                        pages_per_request=c.exact_storage_pages_per_request,
-                        sink_pages=self.exact_fixed_pages,
-                        capacity_tokens=c.pages_per_request * PAGE, **common)
+        _qkv_rope_append(self._append_entry, w["qkv"], x, key_pages=c.exact_key[layer],
+                         value_pages=c.exact_value[layer], key_center=c.key_center[layer],
+                         value_center=c.value_center[layer],
+                         pages_per_request=c.exact_storage_pages_per_request,
+                         sink_pages=self.exact_fixed_pages,
+                         capacity_tokens=c.pages_per_request * PAGE, **common)
 
     def attention(self, layer: int) -> torch.Tensor:
         out = self.attention_output[layer]
@@ -888,7 +944,8 @@ class PageGaugeDecoder:
         c = self.cache
         value_center = c.value_center[layer]
         # with the fused cache update, the decode finalizes a completed page
-        finalize = (self.device_position, c.pages_per_request) if self.fused_append else None
+        finalize = ((self.device_position, c.pages_per_request) if self._append_in_projection
+                    else None)
         if self.tail_attention == "heterogeneous":
             return self.decode.run(self.rotated_query, (c.key_codes[layer], c.value_codes[layer]),
                                    c.key_scales[layer], c.value_scales[layer], c.exact_key[layer],
@@ -907,19 +964,22 @@ class PageGaugeDecoder:
         w = self.weights.layers[layer]
         b = self.batch_size
         qw, kw = cfg.q_heads * DIM, cfg.kv_heads * DIM
-        if self.fused_append:
+        entry = self._projection_entry
+        if self._append_in_projection:
             self._qkv_append(layer)
         else:
-            qkv = projection(w["qkv"], self._hidden, self._qkv, norm_weight=w["input_norm"],
-                             eps=cfg.rms_eps)
+            x, norm = self._norm_input(w["input_norm"])
+            qkv = _projection(entry, w["qkv"], x, self._qkv, norm, cfg.rms_eps, False, None)
             self._append(layer, qkv[:, :qw].view(b, cfg.q_heads, DIM),
                          qkv[:, qw:qw + kw].view(b, cfg.kv_heads, DIM),
                          qkv[:, qw + kw:].view(b, cfg.kv_heads, DIM))
         attended = self.attention(layer)
-        projection(w["o"], attended.view(b, qw), self._hidden, residual=self._hidden)
-        projection(w["gate_up"], self._hidden, self._activation, norm_weight=w["post_norm"],
-                   eps=cfg.rms_eps, swiglu=True)
-        projection(w["down"], self._activation, self._hidden, residual=self._hidden)
+        _projection(entry, w["o"], attended.view(b, qw), self._hidden, None, cfg.rms_eps, False,
+                    self._hidden)
+        x, norm = self._norm_input(w["post_norm"])
+        _projection(entry, w["gate_up"], x, self._activation, norm, cfg.rms_eps, True, None)
+        _projection(entry, w["down"], self._activation, self._hidden, None, cfg.rms_eps, False,
+                    self._hidden)
 
     def _layer(self, layer: int, hidden: torch.Tensor) -> torch.Tensor:
         cfg = self.config
@@ -939,13 +999,16 @@ class PageGaugeDecoder:
         return hidden + F.linear(F.silu(gate) * up, w["down"])
 
     def _body(self, token: torch.Tensor) -> torch.Tensor:
-        if self.fused:
+        if self.fused or self.batched:
             torch.index_select(self.weights.embed, 0, token.reshape(self.batch_size),
                                out=self._hidden)
             for layer in range(self.config.layers):
                 self._layer_fused(layer)
-            return projection(self.weights.lm_head, self._hidden, self._logits,
-                              norm_weight=self.weights.norm, eps=self.config.rms_eps)
+            # larger batches keep returning logits of their own on every step
+            logits = self._logits if self.fused else torch.empty_like(self._logits)
+            x, norm = self._norm_input(self.weights.norm)
+            return _projection(self._projection_entry, self.weights.lm_head, x, logits, norm,
+                               self.config.rms_eps, False, None)
         hidden = F.embedding(token.reshape(self.batch_size), self.weights.embed)
         for layer in range(self.config.layers):
             hidden = self._layer(layer, hidden)
