@@ -11,6 +11,8 @@ import ctypes
 import threading
 from pathlib import Path
 
+import torch
+
 LIBRARY_PATH = Path(__file__).resolve().parent / "lib" / "libpagegauge_hip.so"
 ABI_VERSION = 4
 
@@ -198,6 +200,13 @@ def bench_library():
         if _bench_library is None:
             _bench_library = load_library(BENCH_LIBRARY_PATH, BENCH_PROTOTYPES)
     return _bench_library
+
+
+def current_stream() -> int:
+    """Raw handle of torch's current stream on the current device, without the
+    stream object that ``torch.cuda.current_stream()`` builds (2.5 us a call,
+    a sixth of a small decode call's host time)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def last_error() -> str:

@@ -33,8 +33,7 @@ DIM = 128
 PAGE = 16
 
 
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+_stream = _capi.current_stream
 
 
 def _num_cus(device: torch.device) -> int:
@@ -110,22 +109,24 @@ def _check_page_ids(id_range, pool_pages: int, what: str) -> None:
 def _check_query(q: torch.Tensor, batch: int, num_qo_heads: int) -> None:
     if not q.is_cuda or q.dtype != torch.float16 or q.dim() != 3:
         raise ValueError("q must be a CUDA float16 [B, Hq, 128] tensor")
-    if tuple(q.shape) != (batch, num_qo_heads, DIM):
+    if q.shape != (batch, num_qo_heads, DIM):
         raise ValueError(f"q shape {tuple(q.shape)} does not match the plan ({batch},{num_qo_heads},{DIM})")
-    if q.stride(2) != 1 or q.stride(1) != DIM or q.stride(0) % 8 or q.data_ptr() % 16:
+    batch_stride, head_stride, stride = q.stride()
+    if stride != 1 or head_stride != DIM or batch_stride % 8 or q.data_ptr() % 16:
         raise ValueError("q rows must be contiguous and 16-byte aligned")
 
 
 def _check_cache(cache: torch.Tensor, name: str, dtype: torch.dtype, num_kv_heads: int) -> None:
     if not cache.is_cuda or cache.dtype != dtype or cache.dim() != 4 or not cache.is_contiguous():
         raise ValueError(f"{name} must be a contiguous CUDA {dtype} [pages,16,Hkv,128] tensor")
-    if tuple(cache.shape[1:]) != (PAGE, num_kv_heads, DIM):
+    _, page, heads, dim = cache.shape
+    if page != PAGE or heads != num_kv_heads or dim != DIM:
         raise ValueError(f"{name} must be NHD [pages,16,{num_kv_heads},128]")
 
 
 def _check_scale(scale: torch.Tensor, name: str, pages: int, num_kv_heads: int) -> None:
     if (not scale.is_cuda or scale.dtype != torch.float16 or not scale.is_contiguous()
-            or tuple(scale.shape) != (pages, num_kv_heads)):
+            or scale.shape != (pages, num_kv_heads)):
         raise ValueError(f"{name} must be a contiguous CUDA float16 [{pages},{num_kv_heads}] tensor")
 
 

@@ -158,7 +158,7 @@ def _projection(entry: str, weight: torch.Tensor, x: torch.Tensor, out: torch.Te
                None if norm_weight is None else norm_weight.data_ptr(), float(eps), int(swiglu),
                None if residual is None else residual.data_ptr(),
                0 if residual is None else residual.stride(0), out.data_ptr(), out.stride(0),
-               int(out_f32), torch.cuda.current_stream().cuda_stream)
+               int(out_f32), _capi.current_stream())
     return out
 
 
@@ -234,7 +234,7 @@ def _qkv_rope_append(entry: str, weight, x, norm_weight, eps, query_heads, kv_he
                None if key_center is None else key_center.data_ptr(),
                None if value_center is None else value_center.data_ptr(), center_stride,
                int(pages_per_request), int(sink_pages), int(capacity_tokens),
-               torch.cuda.current_stream().cuda_stream)
+               _capi.current_stream())
 
 
 def argmax_rows(x: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
@@ -248,7 +248,7 @@ def argmax_rows(x: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
     if out.dtype != torch.int64 or out.numel() != x.shape[0] or not out.is_contiguous():
         raise ValueError("argmax output must be contiguous int64 [B]")
     _capi.call("pg_argmax_f32", x.data_ptr(), int(x.shape[0]), int(x.shape[1]), x.stride(0),
-               out.data_ptr(), torch.cuda.current_stream().cuda_stream)
+               out.data_ptr(), _capi.current_stream())
     return out
 
 
@@ -306,7 +306,7 @@ def _causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         _capi.call("pg_causal_attention", q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0),
                    v.data_ptr(), v.stride(0), out.data_ptr(), out.stride(0), int(q.shape[0]),
                    int(q.shape[1]), int(k.shape[1]), 1.0 / math.sqrt(DIM),
-                   torch.cuda.current_stream().cuda_stream)
+                   _capi.current_stream())
         return out
     tokens, hq, _ = q.shape
     hkv = k.shape[1]
@@ -357,7 +357,7 @@ def _norm_rows(x: torch.Tensor, weight: torch.Tensor, eps: float,
     _capi.call("pg_rms_norm", x.data_ptr(), x.stride(0), None if delta is None else delta.data_ptr(),
                0 if delta is None else delta.stride(0), weight.data_ptr(), float(eps),
                out.data_ptr(), out.stride(0), int(x.shape[0]), int(x.shape[1]),
-               torch.cuda.current_stream().cuda_stream)
+               _capi.current_stream())
     return out
 
 
@@ -370,7 +370,7 @@ def _rope_rows(cfg: DecoderConfig, qkv: torch.Tensor, cos: torch.Tensor, sin: to
     k = torch.empty(count, cfg.kv_heads, DIM, device=qkv.device, dtype=qkv.dtype)
     _capi.call("pg_rope_rows", qkv.data_ptr(), qkv.stride(0), cos.data_ptr(), sin.data_ptr(),
                cos.stride(0), q.data_ptr(), k.data_ptr(), count, cfg.q_heads, cfg.kv_heads,
-               torch.cuda.current_stream().cuda_stream)
+               _capi.current_stream())
     return q, k
 
 
@@ -381,7 +381,7 @@ def _swiglu_rows(gate_up: torch.Tensor) -> torch.Tensor:
     rows, width = int(gate_up.shape[0]), int(gate_up.shape[1]) // 2
     out = torch.empty(rows, width, device=gate_up.device, dtype=gate_up.dtype)
     _capi.call("pg_swiglu", gate_up.data_ptr(), gate_up.stride(0), out.data_ptr(), out.stride(0),
-               rows, width, torch.cuda.current_stream().cuda_stream)
+               rows, width, _capi.current_stream())
     return out
 
 

@@ -28,32 +28,46 @@ def _require(condition: bool, message: str) -> None:
         _fail(message)
 
 
+# The checks below first ask for everything at once and go through the
+# conditions one by one (to name the one that fails) only if that does not
+# hold: a launch's checks cost a few microseconds, more than its kernel.
 def _check_tensor(tensor: torch.Tensor, name: str, dtype: torch.dtype, dims: int) -> None:
     # tests/page_gauge_append_extension.cu:23-32
+    if (tensor.is_cuda and tensor.dtype == dtype and tensor.dim() == dims
+            and tensor.is_contiguous()):
+        return
     _require(tensor.is_cuda, f"{name} must be CUDA")
     _require(tensor.dtype == dtype, f"{name} has the wrong dtype")
     _require(tensor.dim() == dims, f"{name} has the wrong rank")
-    _require(tensor.is_contiguous(), f"{name} must be contiguous")
+    _fail(f"{name} must be contiguous")
 
 
 def _check_head_major(tensor: torch.Tensor, name: str) -> None:
     # tests/page_gauge_append_extension.cu:34-41
+    if tensor.is_cuda and tensor.dtype == torch.float16 and tensor.dim() == 3:
+        batch_stride, head_stride, stride = tensor.stride()
+        if (stride == 1 and head_stride == HEAD_DIM and batch_stride % 2 == 0
+                and tensor.data_ptr() % 4 == 0):
+            return
     _require(tensor.is_cuda, f"{name} must be CUDA")
     _require(tensor.dtype == torch.float16, f"{name} must be FP16")
     _require(tensor.dim() == 3, f"{name} must have rank three")
     _require(tensor.stride(2) == 1 and tensor.stride(1) == HEAD_DIM,
              f"{name} must be head-major with a contiguous head dimension")
-    _require(tensor.data_ptr() % 4 == 0 and tensor.stride(0) % 2 == 0,
-             f"{name} rows must be 4-byte aligned")
+    _fail(f"{name} rows must be 4-byte aligned")
 
 
 def _qkv_checks(query, key, value, rotated_query) -> None:
+    q, k = query.shape, key.shape
+    if (q[0] > 0 and q[0] == k[0] and q[2] == HEAD_DIM and k[2] == HEAD_DIM
+            and value.shape == k and rotated_query.shape == q):
+        return
     _require(query.size(0) > 0 and query.size(0) == key.size(0) and query.size(0) == value.size(0),
              "Q/K/V batch sizes must match and be positive")
     _require(query.size(2) == HEAD_DIM and key.size(2) == HEAD_DIM and value.size(2) == HEAD_DIM,
              "head dimension must be 128")
     _require(key.shape == value.shape, "K/V input shapes must match")
-    _require(rotated_query.shape == query.shape, "rotated query shape mismatch")
+    _fail("rotated query shape mismatch")
 
 
 def _check_common(query, key, value, cosine, sine, rotated_query, key_pages, value_pages,
@@ -84,25 +98,28 @@ def _check_dynamic(query, cosine, sine, position) -> None:
     _require(cosine.shape == sine.shape and cosine.size(0) > 0 and cosine.size(1) == HEAD_DIM,
              "dynamic RoPE tables must be matching [positions,128] tensors")
     _require(position.numel() == 1, "dynamic position must contain exactly one int32 scalar")
-    _require(cosine.get_device() == query.get_device() and sine.get_device() == query.get_device()
-             and position.get_device() == query.get_device(),
+    device = query.get_device()
+    _require(cosine.get_device() == device and sine.get_device() == device
+             and position.get_device() == device,
              "dynamic position, RoPE tables, and Q/K/V must share one device")
 
 
 def _check_centers(key_center, value_center, batch: int, kv_heads: int) -> int:
     # tests/page_gauge_append_extension.cu:765-789; returns the center batch stride
+    shape = key_center.shape
+    if (shape == value_center.shape and key_center.is_cuda and value_center.is_cuda
+            and key_center.dtype == torch.float16 and value_center.dtype == torch.float16
+            and key_center.is_contiguous() and value_center.is_contiguous()):
+        if shape == (batch, kv_heads, HEAD_DIM):
+            return kv_heads * HEAD_DIM
+        if batch == 1 and shape == (kv_heads, HEAD_DIM):
+            return 0
     _require(key_center.is_cuda and value_center.is_cuda, "centers must be CUDA")
     _require(key_center.dtype == torch.float16 and value_center.dtype == torch.float16,
              "centers must be FP16")
     _require(key_center.is_contiguous() and value_center.is_contiguous(),
              "centers must be contiguous")
-    shape_ok = key_center.shape == value_center.shape and (
-        (batch == 1 and key_center.dim() == 2 and key_center.size(0) == kv_heads
-         and key_center.size(1) == HEAD_DIM)
-        or (key_center.dim() == 3 and key_center.size(0) == batch
-            and key_center.size(1) == kv_heads and key_center.size(2) == HEAD_DIM))
-    _require(shape_ok, "centers must be [B,Hkv,128] (or [Hkv,128] for batch one)")
-    return 0 if key_center.dim() == 2 else kv_heads * HEAD_DIM
+    _fail("centers must be [B,Hkv,128] (or [Hkv,128] for batch one)")
 
 
 def _check_codes(key_codes, value_codes, key_scales, value_scales, kv_heads: int) -> None:
@@ -110,29 +127,28 @@ def _check_codes(key_codes, value_codes, key_scales, value_scales, kv_heads: int
     _check_tensor(value_codes, "value_codes", torch.int8, 4)
     _check_tensor(key_scales, "key_scales", torch.float16, 2)
     _check_tensor(value_scales, "value_scales", torch.float16, 2)
-    _require(key_codes.shape == value_codes.shape and key_codes.size(1) == PAGE_SIZE
-             and key_codes.size(2) == kv_heads and key_codes.size(3) == HEAD_DIM,
-             "INT8 caches must be NHD [pages,16,Hkv,128]")
+    shape = key_codes.shape
+    _require(shape == value_codes.shape and shape[1] == PAGE_SIZE and shape[2] == kv_heads
+             and shape[3] == HEAD_DIM, "INT8 caches must be NHD [pages,16,Hkv,128]")
 
 
 def _page_gauge_geometry(exact_key_pages, key_codes, key_scales, value_scales, batch: int,
                          kv_heads: int, exact_sink_pages: int) -> tuple[int, int]:
     # tests/page_gauge_append_extension.cu:796-814
-    _require(exact_key_pages.size(0) > 0 and exact_key_pages.size(0) % batch == 0
-             and key_codes.size(0) % batch == 0,
+    ring, codes, scales = exact_key_pages.shape[0], key_codes.shape[0], key_scales.shape
+    _require(ring > 0 and ring % batch == 0 and codes % batch == 0,
              "PageGauge pages must be positive and divide evenly across requests")
-    exact_pages = exact_key_pages.size(0) // batch
+    exact_pages = ring // batch
     _require(exact_sink_pages >= 0, "exact prefix page count must be nonnegative")
     _require(exact_pages > exact_sink_pages, "exact cache must retain at least one tail-ring page")
-    code_pages = key_codes.size(0) // batch
+    code_pages = codes // batch
     _require(exact_sink_pages < code_pages, "exact prefix exceeds the logical cache capacity")
-    _require(key_scales.shape == value_scales.shape and key_scales.size(0) == key_codes.size(0)
-             and key_scales.size(1) == kv_heads, "scales must be [pages,Hkv]")
+    _require(scales == value_scales.shape and scales[0] == codes and scales[1] == kv_heads,
+             "scales must be [pages,Hkv]")
     return exact_pages, code_pages
 
 
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+_stream = _capi.current_stream
 
 
 class PageGaugeAppendExtension:
@@ -241,10 +257,9 @@ class PageGaugeAppendExtension:
         _check_tensor(exact_key_pages, "exact_key_pages", torch.float16, 4)
         _check_tensor(exact_value_pages, "exact_value_pages", torch.float16, 4)
         _qkv_checks(query, key, value, rotated_query)
-        _require(exact_key_pages.shape == exact_value_pages.shape
-                 and exact_key_pages.size(1) == PAGE_SIZE
-                 and exact_key_pages.size(2) == key.size(1)
-                 and exact_key_pages.size(3) == HEAD_DIM,
+        shape = exact_key_pages.shape
+        _require(shape == exact_value_pages.shape and shape[1] == PAGE_SIZE
+                 and shape[2] == key.shape[1] and shape[3] == HEAD_DIM,
                  "exact page cache must be NHD [pages,16,Hkv,128]")
 
     def rope_append_page_gauge_dynamic(self, query, key, value, cosine, sine, position,

@@ -21,8 +21,7 @@ PAGE = 16
 DIM = 128
 
 
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+_stream = _capi.current_stream
 
 
 def _all_cuda_contiguous(*tensors: torch.Tensor) -> None:
