@@ -125,29 +125,18 @@ __device__ __forceinline__ float dot8(v4u_t w, v4u_t x, float acc) {
   return acc;
 }
 
-// Sum of squares of 8 FP16 values in float32.
-__device__ __forceinline__ float squares8(v4u_t x) {
-  const v8h_t h = __builtin_bit_cast(v8h_t, x);
-  float s = 0.0f;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const float f = static_cast<float>(h[e]);
-    s += f * f;
-  }
-  return s;
-}
+// Sum of squares of 8 FP16 values in float32 (v_dot2: exact products).
+__device__ __forceinline__ float squares8(v4u_t x) { return dot8(x, x, 0.0f); }
 
-// MistralRMSNorm of 8 values: fp16(w * fp16(x * inv)).
+// MistralRMSNorm of 8 values: fp16(w * fp16(x * inv)).  The second product is
+// one packed FP16 multiplication: the product of two FP16 values rounded once,
+// as through float32.
 __device__ __forceinline__ v4u_t normalize8(v4u_t x, v4u_t w, float inv) {
   const v8h_t xh = __builtin_bit_cast(v8h_t, x);
-  const v8h_t wh = __builtin_bit_cast(v8h_t, w);
-  v8h_t r;
+  v8h_t n;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const float n = static_cast<float>(static_cast<_Float16>(static_cast<float>(xh[e]) * inv));
-    r[e] = static_cast<_Float16>(static_cast<float>(wh[e]) * n);
-  }
-  return __builtin_bit_cast(v4u_t, r);
+  for (int e = 0; e < 8; ++e) n[e] = static_cast<_Float16>(static_cast<float>(xh[e]) * inv);
+  return __builtin_bit_cast(v4u_t, __builtin_bit_cast(v8h_t, w) * n);
 }
 
 // torch: F.silu(gate) (float32 math, FP16 result) * up (an FP16 product).
@@ -499,24 +488,27 @@ __global__ __launch_bounds__(kGemvThreads) void decoder_gemv_generic_kernel(Gemv
 // of 4 KiB that are refilled one by one, so that the stream does not stop
 // at a tile's reduction.
 //
-// The A operand wants 16 rows x 64 bytes per instruction: half cache lines.
-// Here an instruction loads 8 rows x 128 bytes instead, lanes r < 8 one step
-// of 32 elements and lanes r >= 8 the next, and each step's MFMA uses the half
-// of the operand that belongs to it: twice the MFMAs, half of every result
-// dropped, on units that idle otherwise (28672 x 4096, batch 1: 46.9 us with
-// half lines, 39.5 like this).
+// The operands want 16 rows x 64 bytes per load: half cache lines.  Here a load
+// takes 8 rows x 128 bytes instead, of weights and of inputs, its lanes r < 8
+// one step of 32 elements and the other eight the next: an MFMA then holds
+// the products of 8 weight rows with 8 input rows for both steps, in two
+// quadrants of its result, and the other two are dropped.  That is as many MFMAs
+// as whole operands would need at 16 rows and half as many up to 8 (28672 x
+// 4096, batch 4: 47.8 us with half lines of weights, 39.6 with whole lines of
+// weights, 38.0 with both).
 //
 // kResident (width 4096): a wave's slice of the normalised input stays in
 // registers for all tiles.  Otherwise the input, normalised before the call, is
 // read again with each block of weights (from L2), and any multiple of 512 will
 // do.
 //
-// Cold weights, us for batch 2 / 4 / 16 (v_dot2 kernel for 2 / 4, hipBLASLt
-// without norm and epilogue for 16): QKV 6144 x 4096 13.8 / 13.8 / 15.9 (11.9
-// / 19.5, 17.8), output 4096 x 4096 7.8 / 8.0 / 9.8 (9.1 / 11.8, 17.6),
-// gate/up 28672 x 4096 39.3 / 39.6 / 43.2 (40.5 / 53.7, 60), down 4096 x 14336
-// 20.3 / 21.3 / 28.3 (28.7 / 38.2, 25.7), head 32768 x 4096 44.0 / 44.3 / 46.2
-// (42.7 / 56.2, 58.7).
+// Cold weights, us for batch 2 / 4 / 8 / 16 (v_dot2 kernel for 2 / 4; hipBLASLt
+// without norm and epilogue for 16): QKV 6144 x 4096 12.4 / 12.3 / 12.8 / 15.2
+// (11.9 / 19.5; 18), output 4096 x 4096 7.8 / 7.8 / 8.3 / 9.8 (9.1 / 11.8; 18),
+// gate/up 28672 x 4096 37.8 / 38.0 / 38.5 / 42.3 (40.5 / 53.7; 60), down 4096 x
+// 14336 20.1 / 20.8 / 22.7 / 28.4 (28.7 / 38.2; 25.7), head 32768 x 4096 42.3 /
+// 43.0 / 43.5 / 46.0 (42.7 / 56.2; 58).  At 16 rows the streamed input costs as
+// many bytes from L2 as the weights from HBM.
 // ---------------------------------------------------------------------------
 typedef float v4f_t __attribute__((ext_vector_type(4)));
 constexpr int kTileRows = 16;
@@ -528,8 +520,9 @@ constexpr int kResidentBlocks = 4;   // blocks of a resident slice
 constexpr int kResidentWidth = kMatrixWaves * kMatrixStep * kSteps * kResidentBlocks;   // 4096
 constexpr int kStreamRing = 2;       // blocks in flight with a streamed input
 
-// Sums over the rows' four lanes (16 apart).
-__device__ __forceinline__ float group4_sum(float v) {
+// Sum over the eight lanes of one input row (8, 16 and 32 apart).
+__device__ __forceinline__ float row_lanes_sum(float v) {
+  v += __shfl_xor(v, 8, kWave);
   v += __shfl_xor(v, 16, kWave);
   v += __shfl_xor(v, 32, kWave);
   return v;
@@ -542,31 +535,39 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-template <bool kSwiglu, bool kRope, bool kResident>
+// kHalves: blocks of 8 input rows (1 up to a batch of 8, 2 up to 16).
+template <bool kSwiglu, bool kRope, bool kResident, int kHalves>
 __global__ __launch_bounds__(kWave * kMatrixWaves, kMatrixWaves / 4) void decoder_matrix_kernel(
     GemvArgs a, int batch, int tiles) {
   constexpr bool kPaired = kSwiglu || kRope;      // two weight rows make one output (pair)
   constexpr int kOutRows = kPaired ? kTileRows / 2 : kTileRows;
   constexpr int kRing = kResident ? kResidentBlocks : kStreamRing;   // blocks in flight
-  __shared__ __attribute__((aligned(16))) float partial[2][kMatrixWaves][kTileRows * kMatrixBatch];
-  __shared__ float squares[kMatrixWaves][kMatrixBatch];
+  __shared__ __attribute__((aligned(16))) float partial[2][kMatrixWaves][kTileRows * 8 * kHalves];
+  __shared__ float squares[kMatrixWaves][8 * kHalves];
   __shared__ __attribute__((aligned(16))) uint16_t norm_lds[kResident ? kResidentWidth : 8];
   const int wave = threadIdx.x / kWave;
   const int lane = threadIdx.x % kWave;
-  const int r = lane & 15;             // weight row of the tile (A), input row (B)
+  const int r = lane & 7;              // row of a half, of weights and of inputs
+  const int odd = (lane >> 3) & 1;     // step of a pair
   const int g = lane >> 4;
-  const int steps = kResident ? kResidentBlocks * kSteps : a.k / (kMatrixWaves * kMatrixStep);   // per wave
+  const int steps = kResident ? kResidentBlocks * kSteps : a.k / (kMatrixWaves * kMatrixStep);   // per wave, even
   const int blocks = kResident ? kRing : (steps + kSteps - 1) / kSteps;                // per tile
   const int slice = wave * steps * kMatrixStep + 8 * g;
   const int mine = (tiles - static_cast<int>(blockIdx.x) + static_cast<int>(gridDim.x) - 1) /
                    static_cast<int>(gridDim.x);
-  const uint16_t* x = a.x + min(r, batch - 1) * a.x_stride + slice;
+  const uint16_t* x[kHalves];
+#pragma unroll
+  for (int j = 0; j < kHalves; ++j) x[j] = a.x + min(8 * j + r, batch - 1) * a.x_stride + slice;
 
-  // Block ``block`` (of kSteps steps) of this workgroup's ``count``-th tile.
-  // Register w[s + h] (s even) holds half h of the tile (8 weight rows) for
-  // steps s and s + 1: lanes r < 8 the first, r >= 8 the second, so that an
-  // instruction reads 128 contiguous bytes of each row.
-  auto load = [&](int count, int block, v4u_t (&w)[kSteps]) {
+  // The pair of steps from 2 * i of block ``block`` on, this lane's one of them;
+  // pairs past the slice re-read its last step (no product uses them).
+  auto step_of = [&](int block, int i) {
+    const int step = block * kSteps + 2 * i + odd;
+    return (kResident ? step : min(step, steps - 1)) * kMatrixStep;
+  };
+  // Block ``block`` (of kSteps steps) of this workgroup's ``count``-th tile:
+  // w[h][i] holds half h of the tile for the block's i-th pair of steps.
+  auto load = [&](int count, int block, v4u_t (&w)[2][kSteps / 2]) {
     const int tile = blockIdx.x + count * gridDim.x;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -581,29 +582,22 @@ __global__ __launch_bounds__(kWave * kMatrixWaves, kMatrixWaves / 4) void decode
         first = min(tile * kTileRows + 8 * h, a.out_rows - 1);
         rows = a.out_rows - first;
       }
-      const uint16_t* at = a.weight + static_cast<int64_t>(first) * a.k + min(r & 7, rows - 1) * a.k + slice;
+      const uint16_t* at = a.weight + static_cast<int64_t>(first) * a.k + min(r, rows - 1) * a.k + slice;
 #pragma unroll
-      for (int s = 0; s < kSteps; s += 2) {
-        // a step past the slice re-reads its last one; no product uses it
-        const int step = kResident ? block * kSteps + s + (r >> 3)
-                                   : min(block * kSteps + s + (r >> 3), steps - 1);
-        w[s + h] = __builtin_nontemporal_load(reinterpret_cast<const v4u_t*>(at + step * kMatrixStep));
-      }
+      for (int i = 0; i < kSteps / 2; ++i)
+        w[h][i] = __builtin_nontemporal_load(reinterpret_cast<const v4u_t*>(at + step_of(block, i)));
     }
   };
-  auto load_x = [&](int block, v4u_t (&xv)[kSteps]) {
+  auto load_x = [&](int block, v4u_t (&xv)[kHalves][kSteps / 2]) {
 #pragma unroll
-    for (int s = 0; s < kSteps; ++s) {
-      const int step = kResident ? block * kSteps + s : min(block * kSteps + s, steps - 1);
-      xv[s] = *reinterpret_cast<const v4u_t*>(x + step * kMatrixStep);
-    }
+    for (int j = 0; j < kHalves; ++j)
+#pragma unroll
+      for (int i = 0; i < kSteps / 2; ++i)
+        xv[j][i] = *reinterpret_cast<const v4u_t*>(x[j] + step_of(block, i));
   };
 
-  v4u_t w[kRing][kSteps], xv[kRing][kSteps];
+  v4u_t w[kRing][2][kSteps / 2], xv[kRing][kHalves][kSteps / 2];
   const bool norm = a.norm_weight != nullptr;      // resident only
-  // resident: thread t brings the norm weights 8t..8t+7 to LDS
-  v4u_t norm_part = {0u, 0u, 0u, 0u};
-  if (kResident && norm) norm_part = *reinterpret_cast<const v4u_t*>(a.norm_weight + 8 * threadIdx.x);
   int next_count = 0, next_block = 0;  // the next block to request
   auto advance = [&]() {
     if (++next_block == blocks) {
@@ -611,58 +605,82 @@ __global__ __launch_bounds__(kWave * kMatrixWaves, kMatrixWaves / 4) void decode
       ++next_count;
     }
   };
-#pragma unroll
-  for (int b = 0; b < kRing; ++b) {
-    if constexpr (kResident) {
-      load(0, b, w[b]);
-      load_x(b, xv[b]);
-      __builtin_amdgcn_sched_barrier(0);
-    } else if (next_count < mine) {
-      load(next_count, next_block, w[b]);
-      load_x(next_block, xv[b]);
-      advance();
-    }
-  }
   if constexpr (kResident) {
+    // with a norm the input goes first: loads return in order, and the norm
+    // then runs while the weights arrive
+    v4u_t norm_part = {0u, 0u, 0u, 0u};
     if (norm) {
-      float ss = 0.0f;
+      // thread t brings the norm weights 8t..8t+7 to LDS
+      norm_part = *reinterpret_cast<const v4u_t*>(a.norm_weight + 8 * threadIdx.x);
 #pragma unroll
-      for (int b = 0; b < kRing; ++b)
+      for (int b = 0; b < kRing; ++b) load_x(b, xv[b]);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int s = 0; s < kSteps; ++s) ss += squares8(xv[b][s]);
+      for (int b = 0; b < kRing; ++b) {
+        load(0, b, w[b]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      float ss[kHalves];
+#pragma unroll
+      for (int j = 0; j < kHalves; ++j) {
+        ss[j] = 0.0f;
+#pragma unroll
+        for (int b = 0; b < kRing; ++b)
+#pragma unroll
+          for (int i = 0; i < kSteps / 2; ++i) ss[j] += squares8(xv[b][j][i]);
+        ss[j] = row_lanes_sum(ss[j]);
+        if (lane < 8) squares[wave][8 * j + r] = ss[j];
+      }
       *reinterpret_cast<v4u_t*>(&norm_lds[8 * threadIdx.x]) = norm_part;
-      ss = group4_sum(ss);
-      if (g == 0) squares[wave][r] = ss;
       lds_barrier();
-      float total = 0.0f;
+      float inv[kHalves];
 #pragma unroll
-      for (int i = 0; i < kMatrixWaves; ++i) total += squares[i][r];
-      const float inv = rsqrtf(total / static_cast<float>(a.k) + a.eps);
+      for (int j = 0; j < kHalves; ++j) {
+        float total = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kMatrixWaves; ++i) total += squares[i][8 * j + r];
+        inv[j] = rsqrtf(total / static_cast<float>(a.k) + a.eps);
+      }
 #pragma unroll
       for (int b = 0; b < kRing; ++b) {
 #pragma unroll
-        for (int s = 0; s < kSteps; ++s) {
-          // opaque: the float32 values of the squares are not kept for this
-          // (they would not fit the registers)
-          v4u_t raw = xv[b][s];
-          asm volatile("" : "+v"(raw));
-          xv[b][s] = normalize8(raw, *reinterpret_cast<const v4u_t*>(
-                                         &norm_lds[slice + (b * kSteps + s) * kMatrixStep]), inv);
+        for (int i = 0; i < kSteps / 2; ++i) {
+          const v4u_t nw = *reinterpret_cast<const v4u_t*>(&norm_lds[slice + step_of(b, i)]);
+#pragma unroll
+          for (int j = 0; j < kHalves; ++j) xv[b][j][i] = normalize8(xv[b][j][i], nw, inv[j]);
         }
         __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+#pragma unroll
+      for (int b = 0; b < kRing; ++b) {
+        load(0, b, w[b]);
+        load_x(b, xv[b]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int b = 0; b < kRing; ++b) {
+      if (next_count < mine) {
+        load(next_count, next_block, w[b]);
+        load_x(next_block, xv[b]);
+        advance();
       }
     }
   }
 
-  // acc[h][j]: half h of the tile with steps of parity j.  Its valid rows are
-  // those whose lanes held that step: C rows 8j..8j+7.
-  v4f_t acc[2][2];
+  // acc[h][j]: half h of the tile with half j of the batch.  A lane's operands
+  // belong to one step of the pair, so the products of C rows m and columns n
+  // are valid where both are below 8 (even steps) or both are not (odd steps).
+  v4f_t acc[2][kHalves];
 #pragma unroll
   for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[h][j] = v4f_t{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int j = 0; j < kHalves; ++j) acc[h][j] = v4f_t{0.0f, 0.0f, 0.0f, 0.0f};
   AppendInputs append_in{};
-  auto compute = [&](int count, int block, v4u_t (&wb)[kSteps], v4u_t (&xb)[kSteps]) {
+  auto compute = [&](int count, int block, v4u_t (&wb)[2][kSteps / 2],
+                     v4u_t (&xb)[kHalves][kSteps / 2]) {
     const int tile = blockIdx.x + count * gridDim.x;
     if constexpr (kRope) {
       // the row pairs' RoPE / center inputs, requested before the products
@@ -670,28 +688,34 @@ __global__ __launch_bounds__(kWave * kMatrixWaves, kMatrixWaves / 4) void decode
         append_in = append_inputs(a, threadIdx.x / 8, tile * 8 + threadIdx.x % 8);
     }
 #pragma unroll
-    for (int s = 0; s < kSteps; ++s) {
-      if (!kResident && block * kSteps + s >= steps) break;
+    for (int i = 0; i < kSteps / 2; ++i) {
+      if (!kResident && block * kSteps + 2 * i >= steps) break;
 #pragma unroll
       for (int h = 0; h < 2; ++h)
-        acc[h][s & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-            __builtin_bit_cast(v8h_t, wb[(s & ~1) + h]), __builtin_bit_cast(v8h_t, xb[s]),
-            acc[h][s & 1], 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < kHalves; ++j)
+          acc[h][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+              __builtin_bit_cast(v8h_t, wb[h][i]), __builtin_bit_cast(v8h_t, xb[j][i]), acc[h][j],
+              0, 0, 0);
     }
     if (block != blocks - 1) return;
-    // lane (input row r): rows 4 (g % 2).. of half h, the even steps' sum where
-    // g < 2 and the odd steps' where g >= 2; the two are added, and lanes g
-    // keep rows 4g..4g+3 of the tile
-    v4f_t sum[2];
+    // even and odd steps' sums of C row m and column n sit 8 columns and 8 rows
+    // (lanes 8 + 32) apart; of each pair of lanes with valid sums, the lower
+    // keeps half 0 of the tile and the upper half 1, rows 4 (g % 2).. of it
+    float (&sums)[kMatrixWaves][kTileRows * 8 * kHalves] = partial[count & 1];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const v4f_t own = g < 2 ? acc[h][0] : acc[h][1];
+    for (int j = 0; j < kHalves; ++j) {
+      v4f_t sum;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) sum[h][e] = own[e] + __shfl_xor(own[e], 32, kWave);
-      acc[h][0] = acc[h][1] = v4f_t{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int e = 0; e < 4; ++e) {
+        const float s0 = acc[0][j][e] + __shfl_xor(acc[0][j][e], 40, kWave);
+        const float s1 = acc[1][j][e] + __shfl_xor(acc[1][j][e], 40, kWave);
+        sum[e] = odd ? s1 : s0;
+      }
+      if ((g >> 1) == odd)
+        *reinterpret_cast<v4f_t*>(&sums[wave][(8 * j + r) * kTileRows + 8 * odd + 4 * (g & 1)]) = sum;
+      acc[0][j] = acc[1][j] = v4f_t{0.0f, 0.0f, 0.0f, 0.0f};
     }
-    float (&sums)[kMatrixWaves][kTileRows * kMatrixBatch] = partial[count & 1];
-    *reinterpret_cast<v4f_t*>(&sums[wave][r * kTileRows + 4 * g]) = g < 2 ? sum[0] : sum[1];
     lds_barrier();
     // a thread per output: input row b, output row o of the tile
     const int b = threadIdx.x / kOutRows;
@@ -713,7 +737,7 @@ __global__ __launch_bounds__(kWave * kMatrixWaves, kMatrixWaves / 4) void decode
   if constexpr (kResident) {
     // two tiles in turn, a block's registers refilled two tiles ahead as soon
     // as its products are done
-    v4u_t w2[kRing][kSteps];
+    v4u_t w2[kRing][2][kSteps / 2];
     if (mine > 1) {
 #pragma unroll
       for (int b = 0; b < kRing; ++b) {
@@ -761,27 +785,30 @@ __global__ __launch_bounds__(kWave * kMatrixWaves, kMatrixWaves / 4) void decode
 
 constexpr int kMatrixBlocks = 256;   // one 16-wave workgroup per CU
 
-// Batches the matrix kernel takes; a.swiglu / ``rope`` pick the epilogue.
-template <bool kRope>
-int32_t launch_matrix(const GemvArgs& a, int batch, hipStream_t s, const char* what) {
-  const int per_tile = a.swiglu || kRope ? kTileRows / 2 : kTileRows;
-  const int rows = kRope ? a.out_rows / 2 : a.out_rows;
-  const int tiles = (rows + per_tile - 1) / per_tile;
+template <bool kSwiglu, bool kRope>
+void launch_matrix_kernel(const GemvArgs& a, int batch, int tiles, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>(tiles < kMatrixBlocks ? tiles : kMatrixBlocks));
   const auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, dim3(kWave * kMatrixWaves), 0, s, a, batch, tiles);
   };
   const bool resident = a.k == kResidentWidth;
-  if constexpr (kRope) {
-    if (resident) launch(decoder_matrix_kernel<false, true, true>);
-    else launch(decoder_matrix_kernel<false, true, false>);
-  } else if (a.swiglu) {
-    if (resident) launch(decoder_matrix_kernel<true, false, true>);
-    else launch(decoder_matrix_kernel<true, false, false>);
+  if (batch <= 8) {
+    if (resident) launch(decoder_matrix_kernel<kSwiglu, kRope, true, 1>);
+    else launch(decoder_matrix_kernel<kSwiglu, kRope, false, 1>);
   } else {
-    if (resident) launch(decoder_matrix_kernel<false, false, true>);
-    else launch(decoder_matrix_kernel<false, false, false>);
+    if (resident) launch(decoder_matrix_kernel<kSwiglu, kRope, true, 2>);
+    else launch(decoder_matrix_kernel<kSwiglu, kRope, false, 2>);
   }
+}
+
+// a.swiglu / ``kRope`` pick the epilogue.
+template <bool kRope>
+int32_t launch_matrix(const GemvArgs& a, int batch, hipStream_t s, const char* what) {
+  const int per_tile = a.swiglu || kRope ? kTileRows / 2 : kTileRows;
+  const int rows = kRope ? a.out_rows / 2 : a.out_rows;
+  const int tiles = (rows + per_tile - 1) / per_tile;
+  if (!kRope && a.swiglu) launch_matrix_kernel<true, false>(a, batch, tiles, s);
+  else launch_matrix_kernel<false, kRope>(a, batch, tiles, s);
   return check_launch(what);
 }
 
