@@ -110,7 +110,7 @@ int32_t build_plan(const int32_t* host_indptr, const int32_t* host_last_page_len
                    int32_t head_dim, int32_t page_size, int32_t split_pages,
                    int32_t tail_split_pages, int32_t exact_tail_pages_hint, int32_t num_cus,
                    std::vector<WorkItem>& items, std::vector<int32_t>& item_ptr,
-                   pg_decode_plan_t& p) {
+                   pg_decode_plan_t& p, bool fewest_items) {
   if (!host_indptr || !host_last_page_len)
     return fail(PG_ERROR_INVALID_ARGUMENT, "null plan argument");
   if (batch_size <= 0) return fail(PG_ERROR_INVALID_ARGUMENT, "batch size must be positive");
@@ -204,7 +204,7 @@ int32_t build_plan(const int32_t* host_indptr, const int32_t* host_last_page_len
       }
       return total;
     };
-    double lo = 1e-3, hi = 1.0;
+    double lo, hi = 1.0;
     for (const Segment& sg : segments) hi += (sg.end - sg.begin) * sg.weight;
     // Measured on MI355X (B=1 sweeps from 4K to 160K tokens, B=4 and B=8):
     // * large (>= 30 pages per CU): 16-page chunks beat finer ones, because
@@ -217,14 +217,44 @@ int32_t build_plan(const int32_t* host_indptr, const int32_t* host_last_page_len
     //   item cap needs more than 128 items, a second wave of workgroups;
     // * small: chunks down to one PV group for parallelism.
     const double per_cu = hi / static_cast<double>(target);
+    const double whole = hi;
+    const int64_t most_uncut = count_for(whole, nullptr);   // the 64-page cap's own items
     medium = per_cu >= 3.0 && per_cu < kMediumMaxPagesPerCu;
-    const int64_t item_target = medium ? std::max<int64_t>(1, target * 7 / 16) : target;
+    // A fuller plan than these regimes ask for, where the 64-page cap or the
+    // raggedness of a batch leaves the last round of workgroups nearly empty.
+    // Not where it could pass the limit of items per request.
+    const bool fuller = !fewest_items && per_cu >= 3.0 && target * 3 / 2 <= kMaxItemsPerRequest;
+    // More than half the CUs in uncut items: at two workgroups per item a
+    // medium plan would start a second round for the few that are left over
+    // (142 items, FP16 B56: 119 us; 256 items: 97 us).
+    if (fuller && most_uncut * 2 > target) medium = false;
     lo = per_cu >= kMediumMaxPagesPerCu ? kLargeBatchMinChunk : 1e-3;
-    if (count_for(hi, nullptr) <= item_target) {
-      for (int iter = 0; iter < 64; ++iter) {
-        const double mid = 0.5 * (lo + hi);
-        if (count_for(mid, nullptr) <= item_target) hi = mid; else lo = mid;
+    auto balance = [&](int64_t item_target) {
+      double low = lo, high = whole;
+      if (most_uncut <= item_target) {
+        for (int iter = 0; iter < 64; ++iter) {
+          const double mid = 0.5 * (low + high);
+          if (count_for(mid, nullptr) <= item_target) high = mid; else low = mid;
+        }
       }
+      return high;
+    };
+    hi = balance(medium ? std::max<int64_t>(1, target * 7 / 16) : target);
+    if (fuller && !medium && (most_uncut <= target || !host_tail_indptr)) {
+      // The heaviest item of one round carries over 5/4 of a CU's share (or
+      // the uncut items pass one round): three half-size workgroups for every
+      // two that run at a time even the load out.  B15 x 19K FP16, 285 items:
+      // 225 us, 375: 204 us; B18 x 16K heterogeneous, 312 items: 124 us, 384:
+      // 118 us; B95 x 1.5K FP16, 256 items: 117 us, 380: 110 us.  An even
+      // round is the better one (B8 ragged, 256 items: 64 us, 384: 67 us).
+      // Segmented plans whose uncut items pass one round keep those items.
+      std::vector<int> cut(segments.size(), 0);
+      count_for(hi, &cut);
+      double heaviest = 0.0;
+      for (size_t i = 0; i < segments.size(); ++i)
+        heaviest = std::max(heaviest, std::ceil(static_cast<double>(segments[i].end - segments[i].begin) /
+                                                cut[i]) * segments[i].weight);
+      if (most_uncut > target || heaviest > 1.25 * per_cu) hi = balance(target * 3 / 2);
     }
     count_for(hi, &chunks);
   }

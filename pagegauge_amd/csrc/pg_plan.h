@@ -85,14 +85,16 @@ int waves_per_block_for(int hkv, int64_t items, int64_t num_cus);
 
 // Host half of the planner: validates the batch and cuts it into work items
 // (``items``, ``item_ptr`` [B+1]).  Fills ``p``; the caller checks the
-// workspace size and copies the work list to the device.
+// workspace size and copies the work list to the device.  ``fewest_items``:
+// the regimes' own item counts, without the fuller rounds, for a workspace
+// that the fuller plan does not fit.
 int32_t build_plan(const int32_t* host_indptr, const int32_t* host_last_page_len,
                    int32_t batch_size, int32_t primary_kind, const int32_t* host_tail_indptr,
                    const int32_t* host_tail_last_len, int32_t num_qo_heads, int32_t num_kv_heads,
                    int32_t head_dim, int32_t page_size, int32_t split_pages,
                    int32_t tail_split_pages, int32_t exact_tail_pages_hint, int32_t num_cus,
                    std::vector<WorkItem>& items, std::vector<int32_t>& item_ptr,
-                   pg_decode_plan_t& p);
+                   pg_decode_plan_t& p, bool fewest_items = false);
 
 // Device dispatch order of a plan's items: with more items than CUs
 // (several rounds of workgroups), the heaviest items first, by the weight
