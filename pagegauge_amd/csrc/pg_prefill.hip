@@ -71,7 +71,9 @@ struct AttentionArgs {
 //
 // The running maximum is raised only when a score exceeds it by more than
 // 2^8 (probabilities then reach 256, which FP16 holds at the same relative
-// precision): most tiles skip the rescale of the accumulators.
+// precision): most tiles skip the rescale of the accumulators.  A lane adds its
+// probabilities in float32, in two sums: half the chain, half the terms in each
+// (16384 tokens 2036 us with one, 2032 with two; 1000 tokens 22.8 both).
 //
 // Blocks are dispatched longest first, and KV heads vary fastest, so that with
 // 8 heads each XCD works on one head's keys and values.
@@ -150,7 +152,7 @@ __global__ __launch_bounds__(kWave * kWaves, 2) void causal_attention_kernel(Att
   for (int d = 0; d < 4; ++d)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[d][r] = 0.0f;
-  float m = kNegInf, l = 0.0f;
+  float m = kNegInf, l = 0.0f, l1 = 0.0f;
 
   auto qk = [&](int buffer, v16f (&s)[2]) {
 #pragma unroll
@@ -181,6 +183,7 @@ __global__ __launch_bounds__(kWave * kWaves, 2) void causal_attention_kernel(Att
       const float alpha = __builtin_amdgcn_exp2f(m - m_new);
       m = m_new;
       l *= alpha;
+      l1 *= alpha;
 #pragma unroll
       for (int d = 0; d < 4; ++d)
 #pragma unroll
@@ -193,7 +196,7 @@ __global__ __launch_bounds__(kWave * kWaves, 2) void causal_attention_kernel(Att
         const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[b][r], a.scale_log2, -m));
         const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[b][r + 1], a.scale_log2, -m));
         l += p0;
-        l += p1;
+        l1 += p1;
         p[2 * b + r / 8][r % 8] = static_cast<_Float16>(p0);
         p[2 * b + r / 8][r % 8 + 1] = static_cast<_Float16>(p1);
       }
@@ -262,6 +265,7 @@ __global__ __launch_bounds__(kWave * kWaves, 2) void causal_attention_kernel(Att
   }
 
   {
+    l += l1;
     const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
     l = __uint_as_float(x[0]) + __uint_as_float(x[1]);
   }
