@@ -11,9 +11,10 @@
 // default correctly rounded division), and the sign-symmetric
 // floor(q + 0.5f) rounding is evaluated in float32 exactly as written.
 //
-// Layout per launch: one wave64 per (request, head row); lane l owns the two
-// adjacent dimensions 2l and 2l+1, so every row access is one coalesced
-// 256-byte (FP16) or 128-byte (INT8) transaction per wave.
+// Layout of the append kernels: one wave64 per (request, head row); lane l
+// owns the two adjacent dimensions 2l and 2l+1, so every row access is one
+// coalesced 256-byte (FP16) or 128-byte (INT8) transaction per wave.  The bulk
+// quantizer and the centers read 16 bytes per lane (their own comments).
 #pragma clang fp contract(off)
 
 #include "pg_common.h"

@@ -12,7 +12,10 @@ Per decode step and layer (``_layer``):
   center, one partial kernel and one combine kernel) -> output projection ->
   residual -> RMSNorm -> fused gate/up -> SiLU * up -> down -> residual.
 
-Everything but K1/K2 is plain PyTorch-ROCm (fp16 GEMMs on hipBLASLt).  The
+A step's projections run on hand-written kernels with their element-wise
+neighbours (``pg_decoder_gemv`` for one row, ``pg_decoder_gemm`` on the matrix
+cores for 2 to 16); other sizes run on torch operators.  A prompt's attention,
+norms, RoPE and SwiGLU are HIP kernels between fp16 GEMMs on hipBLASLt.  The
 ``"fp16"`` backend is the same decoder over an FP16 paged cache
 (``rope_append_fp16_dynamic`` + the same-way FP16 decode kernel): the
 reference's ``flashinfer_fp16`` baseline.
@@ -748,8 +751,8 @@ class PageGaugeDecoder:
         self.graph_replays = 0
         self.eager_steps = 0
         self.graph_bank_misses = 0
-        # fused projections (pg_decoder_gemv): batch <= 4, widths multiples of
-        # 512, and batch * width <= 32768 unless the width is 4096 or 14336
+        # fused projections: batch <= 4 (``projection`` picks pg_decoder_gemv or,
+        # from 2 rows on, the matrix cores), widths multiples of 512, and batch * width <= 32768 unless the width is 4096 or 14336
         ok = batch_size <= 4 and all(
             w % 512 == 0 and (w in (4096, 14336) or batch_size * w <= 32768)
             for w in (cfg.hidden, cfg.intermediate))
