@@ -783,7 +783,7 @@ __global__ __launch_bounds__(kWave * kMatrixWaves, kMatrixWaves / 4) void decode
   }
 }
 
-constexpr int kMatrixBlocks = 256;   // one 16-wave workgroup per CU
+constexpr int kMatrixBlocks = 256;   // one workgroup of 8 waves per CU
 
 template <bool kSwiglu, bool kRope>
 void launch_matrix_kernel(const GemvArgs& a, int batch, int tiles, hipStream_t s) {

@@ -231,8 +231,9 @@ def _qkv_rope_append(entry: str, weight, x, norm_weight, eps, query_heads, kv_he
     stride = 1 if positions.numel() == batch and batch > 1 else 0
     center_stride = 0 if key_center is None else kv_heads * DIM
     _capi.call(entry, weight.data_ptr(), k, x.data_ptr(), x.stride(0),
-               batch, None if norm_weight is None else norm_weight.data_ptr(), float(eps), query_heads, kv_heads, cos.data_ptr(),
-               sin.data_ptr(), cos.stride(0), int(cos.shape[0]), positions.data_ptr(), stride,
+               batch, None if norm_weight is None else norm_weight.data_ptr(), float(eps),
+               query_heads, kv_heads, cos.data_ptr(), sin.data_ptr(), cos.stride(0),
+               int(cos.shape[0]), positions.data_ptr(), stride,
                rotated_query.data_ptr(), key_pages.data_ptr(), value_pages.data_ptr(),
                None if key_center is None else key_center.data_ptr(),
                None if value_center is None else value_center.data_ptr(), center_stride,
@@ -751,8 +752,9 @@ class PageGaugeDecoder:
         self.graph_replays = 0
         self.eager_steps = 0
         self.graph_bank_misses = 0
-        # fused projections: batch <= 4 (``projection`` picks pg_decoder_gemv or,
-        # from 2 rows on, the matrix cores), widths multiples of 512, and batch * width <= 32768 unless the width is 4096 or 14336
+        # fused projections (pg_decoder_gemv, which goes to the matrix cores where
+        # they are faster): batch <= 4, widths multiples of 512, and
+        # batch * width <= 32768 unless the width is 4096 or 14336
         ok = batch_size <= 4 and all(
             w % 512 == 0 and (w in (4096, 14336) or batch_size * w <= 32768)
             for w in (cfg.hidden, cfg.intermediate))
