@@ -521,13 +521,11 @@ class GaugeCache:
         self.exact_value = torch.zeros_like(self.exact_key)
         self.pages_per_request = pages
         self.batch_size = batch_size
-        self._center_workspace: Optional[torch.Tensor] = None
 
     def clone(self) -> "GaugeCache":
         other = GaugeCache.__new__(GaugeCache)
         for name, value in vars(self).items():
             setattr(other, name, value.clone() if isinstance(value, torch.Tensor) else value)
-        other._center_workspace = None
         return other
 
     def populate(self, layer: int, request: int, key: torch.Tensor, value: torch.Tensor) -> None:
@@ -535,7 +533,9 @@ class GaugeCache:
         centers, INT8 codes and scales of every page, and the centered FP16
         copies of its exact pages (the sink prefix, the static suffix and the
         last tail pages) in their slots
-        (diagnostics/benchmark_backend_exclusive.py:427-506)."""
+        (diagnostics/benchmark_backend_exclusive.py:427-506).  Asynchronous on
+        the current stream; calls for different layers or requests may run on
+        different streams at once."""
         tokens = key.shape[0]
         pages = tokens // PAGE
         if tokens % PAGE or pages > self.pages_per_request:
@@ -544,12 +544,11 @@ class GaugeCache:
             raise ValueError("fixture must contain at least one quantized old page")
         if self.exact_static_suffix_pages and pages < self.initial_context_pages:
             raise ValueError("the static suffix lies beyond the cached prefix")
-        from . import _capi
-        need = int(_capi.library().pg_token_major_centers_workspace_bytes(tokens, key.shape[1]))
-        if self._center_workspace is None or self._center_workspace.numel() < need:
-            self._center_workspace = torch.empty(need, device=key.device, dtype=torch.uint8)
         kc, vc = self.key_center[layer, request], self.value_center[layer, request]
-        token_major_centers(key, value, kc, vc, self._center_workspace)
+        # the chunk sums' scratch is the call's own, from the allocator, which
+        # orders its reuse by stream: nothing here waits for the GPU, so that
+        # populates on other streams may be running beside this one
+        token_major_centers(key, value, kc, vc)
         layout = pt.ExactPageLayout.checked(self.exact_sink_pages, self.exact_static_suffix_pages,
                                             self.initial_context_pages, self.exact_tail_pages)
         base = request * self.pages_per_request
