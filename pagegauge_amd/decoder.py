@@ -332,18 +332,33 @@ def _causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     return out
 
 
+def _shaped_as_configured(weights: DecoderWeights) -> bool:
+    """Every weight has exactly its configured shape.  The kernels take sizes
+    from the configuration and pointers from the weights; a shape that torch
+    operators broadcast (a norm weight of one element) or refuse is theirs."""
+    cfg = weights.config
+    h, i = cfg.hidden, cfg.intermediate
+    shapes = {"input_norm": (h,), "qkv": (cfg.qkv_width, h), "o": (h, cfg.q_heads * DIM),
+              "post_norm": (h,), "gate_up": (2 * i, h), "down": (h, i)}
+    return (weights.norm.shape == (h,)
+            and all(w.dim() == 2 and w.shape[1] == h for w in (weights.embed, weights.lm_head))
+            and all(layer[name].shape == shape for layer in weights.layers
+                    for name, shape in shapes.items()))
+
+
 def _prefill_kernels_take(weights: DecoderWeights, tokens: torch.Tensor, cos: torch.Tensor,
                           sin: torch.Tensor) -> bool:
     """Whether ``prefill`` runs its element-wise work as HIP kernels: FP16
-    weights and dense 16-byte aligned RoPE rows on the current device, widths
-    that the kernels read (multiples of 8; norms up to 16384).  The GEMMs'
-    inputs and outputs are fresh tensors, dense and aligned."""
+    weights of the configured shapes and dense 16-byte aligned RoPE rows on the
+    current device, widths that the kernels read (multiples of 8; norms up to
+    16384).  The GEMMs' inputs and outputs are fresh tensors, dense and
+    aligned."""
     cfg = weights.config
     return (tokens.numel() > 0 and cfg.hidden % 8 == 0 and cfg.hidden <= 16384
             and cfg.intermediate % 8 == 0 and tokens.numel() <= min(cos.shape[0], sin.shape[0])
             and _on_current_device(weights.embed, weights.norm, weights.lm_head, cos, sin,
                                    *(w for layer in weights.layers for w in layer.values()))
-            and tokens.device == weights.embed.device
+            and tokens.device == weights.embed.device and _shaped_as_configured(weights)
             and all(t.dim() == 2 and t.shape[1] == DIM and t.stride(1) == 1
                     and t.stride(0) % 8 == 0 and t.stride(0) >= DIM and t.data_ptr() % 16 == 0
                     for t in (cos, sin))
@@ -357,6 +372,11 @@ def _norm_rows(x: torch.Tensor, weight: torch.Tensor, eps: float,
     """``rms_norm(x + delta)``, the sum left in ``x``, in one HIP launch."""
     from . import _capi
 
+    if (weight.shape != x.shape[1:] or weight.dtype != x.dtype or weight.device != x.device
+            or not weight.is_contiguous()):
+        raise ValueError("norm weight must be contiguous FP16 [K]")
+    if delta is not None and delta.shape != x.shape:
+        raise ValueError("the residual must be shaped like the rows")
     out = torch.empty_like(x)
     _capi.call("pg_rms_norm", x.data_ptr(), x.stride(0), None if delta is None else delta.data_ptr(),
                0 if delta is None else delta.stride(0), weight.data_ptr(), float(eps),
@@ -786,19 +806,19 @@ class PageGaugeDecoder:
     def _matrix_projections_take(weights: DecoderWeights, batch_size: int) -> bool:
         """``pg_decoder_gemm`` takes up to 16 rows, widths that are multiples
         of 512 (up to 16384 for the norm) and contiguous 16-byte aligned FP16
-        weights.  At widths other than 4096 every tile of weights re-reads the
-        input, which torch operators overtake as batch x width grows (four
-        layers and head, batch 16: 5120 wide 850 us against 1158 in torch
-        operators, 8192 wide 1839 against 1755; batch 8, 8192 wide 1513
-        against 1714)."""
+        weights of the configured shapes.  At widths other than 4096 every tile
+        of weights re-reads the input, which torch operators overtake as batch
+        x width grows (four layers and head, batch 16: 5120 wide 850 us against
+        1158 in torch operators, 8192 wide 1839 against 1755; batch 8, 8192
+        wide 1513 against 1714)."""
         cfg = weights.config
         if cfg.hidden != 4096 and batch_size * cfg.hidden > 98304:
             return False
         tensors = [weights.embed, weights.norm, weights.lm_head,
                    *(t for layer in weights.layers for t in layer.values())]
         return (batch_size <= 16 and cfg.hidden % 512 == 0 and cfg.hidden <= 16384
-                and cfg.intermediate % 512 == 0
-                and _on_current_device(*tensors)
+                and cfg.intermediate % 512 == 0 and _shaped_as_configured(weights)
+                and weights.lm_head.shape[0] == cfg.vocab and _on_current_device(*tensors)
                 and all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in tensors))
 
     # -- plan --------------------------------------------------------------
