@@ -450,8 +450,11 @@ extern "C" int32_t pg_causal_attention(const void* query, int64_t query_stride, 
   clear_error();
   if (!query || !key || !value || !out) return fail(PG_ERROR_INVALID_ARGUMENT, "null tensor pointer");
   if (tokens <= 0) return fail(PG_ERROR_INVALID_ARGUMENT, "the prompt must hold at least one token");
-  if (kv_heads <= 0 || query_heads != kGqa * kv_heads)
+  if (kv_heads <= 0 || query_heads != static_cast<int64_t>(kGqa) * kv_heads)
     return fail(PG_ERROR_UNSUPPORTED, "the attention kernel requires GQA group size 4");
+  // key and block numbers are int32, up to a block past the last token
+  if (tokens > 0x7fffffff - 64 || (static_cast<int64_t>(tokens) + 31) / 32 * kv_heads > 0x7fffffff)
+    return fail(PG_ERROR_INVALID_ARGUMENT, "too many tokens");
   const int64_t q_row = static_cast<int64_t>(query_heads) * kHeadDim;
   const int64_t kv_row = static_cast<int64_t>(kv_heads) * kHeadDim;
   if (query_stride < q_row || out_stride < q_row || key_stride < kv_row || value_stride < kv_row ||
@@ -526,7 +529,10 @@ extern "C" int32_t pg_rope_rows(const void* qkv, int64_t qkv_stride, const void*
     return fail(PG_ERROR_INVALID_ARGUMENT, "null tensor pointer");
   if (tokens <= 0 || query_heads <= 0 || kv_heads <= 0)
     return fail(PG_ERROR_INVALID_ARGUMENT, "tokens and head counts must be positive");
-  if (qkv_stride < static_cast<int64_t>(query_heads + kv_heads) * kHeadDim || qkv_stride % 8 ||
+  const int64_t heads = static_cast<int64_t>(query_heads) + kv_heads;
+  if (heads > 0x7fffffff / kHeadDim || tokens > 0x7fffffffffff / (heads * 8))
+    return fail(PG_ERROR_INVALID_ARGUMENT, "too many tokens");
+  if (qkv_stride < heads * kHeadDim || qkv_stride % 8 ||
       rope_stride < kHeadDim || rope_stride % 8 || !aligned(qkv, 16) || !aligned(cosine, 16) ||
       !aligned(sine, 16) || !aligned(query, 16) || !aligned(key, 16))
     return fail(PG_ERROR_INVALID_ARGUMENT, "rows must be 16-byte aligned and their strides cover the heads");
@@ -540,7 +546,7 @@ extern "C" int32_t pg_rope_rows(const void* qkv, int64_t qkv_stride, const void*
   a.key = static_cast<uint16_t*>(key);
   a.query_heads = query_heads;
   a.kv_heads = kv_heads;
-  a.units = tokens * (query_heads + kv_heads) * 8;
+  a.units = tokens * heads * 8;
   const int64_t blocks = (a.units + kRowThreads - 1) / kRowThreads;
   if (blocks > 0x7fffffff) return fail(PG_ERROR_INVALID_ARGUMENT, "too many tokens");
   hipLaunchKernelGGL(rope_rows_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kRowThreads), 0,

@@ -379,7 +379,7 @@ __device__ __forceinline__ int64_t exact_slot(const QuantizeParams& p, int64_t p
   if (p.exact_map != nullptr) return p.exact_map[page];
   if (p.tail_pages <= 0) return -1;
   if (page < p.sink_pages) return p.first_slot + page;
-  if (page >= p.suffix_begin && page < p.suffix_begin + p.suffix_pages)
+  if (page >= p.suffix_begin && page - p.suffix_begin < p.suffix_pages)
     return p.first_slot + p.sink_pages + (page - p.suffix_begin);
   if (page >= p.num_pages - p.tail_pages)
     return p.first_slot + p.sink_pages + p.suffix_pages + page % p.tail_pages;
@@ -1083,12 +1083,14 @@ extern "C" int32_t pg_prefill_page_gauge_layout(
   clear_error();
   if (!exact_key_pages || !exact_value_pages)
     return fail(PG_ERROR_INVALID_ARGUMENT, "null tensor pointer");
-  if (sink_pages < 0 || suffix_begin < 0 || suffix_pages < 0 || tail_pages <= 0 || first_slot < 0)
+  if (sink_pages < 0 || suffix_begin < 0 || suffix_pages < 0 || tail_pages <= 0 || first_slot < 0 ||
+      num_exact_pages < 0)
     return fail(PG_ERROR_INVALID_ARGUMENT,
                 "the exact layout needs non-negative fixed pages and a tail ring");
   if (suffix_pages > 0 && suffix_begin < sink_pages)
     return fail(PG_ERROR_INVALID_ARGUMENT, "the static suffix must lie behind the prefix");
-  if (first_slot + sink_pages + suffix_pages + tail_pages > num_exact_pages)
+  // first_slot on the other side: the sum of int64 arguments could wrap
+  if (first_slot > num_exact_pages - (int64_t{sink_pages} + suffix_pages + tail_pages))
     return fail(PG_ERROR_INVALID_ARGUMENT, "the exact layout points past the exact pages");
   QuantizeParams p{};
   if (int32_t rc = prefill_params(key, key_token_stride, value, value_token_stride, key_center,

@@ -257,3 +257,42 @@ def test_read_probes_reject_a_short_sink():
     assert "an entry per workgroup (512 > 511)" in lib.pg_last_error().decode()
     assert lib.pg_probe_page_walk(fake, fake, fake, 40, 4, 16384, fake, 9, None, None, None) == 1
     assert "(10 > 9)" in lib.pg_last_error().decode()
+
+
+MOST = 2 ** 63 - 1
+
+
+@pytest.mark.parametrize("over,message", [
+    (dict(first_slot=16), "past the exact pages"),
+    (dict(first_slot=MOST), "past the exact pages"),
+    (dict(first_slot=MOST - 15), "past the exact pages"),
+    (dict(sink=2 ** 31 - 1, suffix_begin=2 ** 31 - 1, suffix=2 ** 31 - 1), "past the exact pages"),
+    (dict(num_exact=0), "past the exact pages"),
+])
+def test_prefill_layout_rejects_slots_past_the_pool(over, message):
+    """Slot numbers whose sums leave int64 or int32 among them."""
+    a = dict(key=FAKE, key_stride=1024, value=FAKE, value_stride=1024, key_center=FAKE,
+             value_center=FAKE, key_codes=FAKE, value_codes=FAKE, key_scales=FAKE,
+             value_scales=FAKE, exact_key=FAKE, exact_value=FAKE, num_exact=16, first_slot=0,
+             sink=0, suffix_begin=0, suffix=0, tail=16, pages=40, heads=8, stream=None)
+    a.update(over)
+    rc, text = _call("pg_prefill_page_gauge_layout", *a.values())
+    assert rc == 1 and message in text
+
+
+@pytest.mark.parametrize("tokens,kv_heads,message", [
+    (2 ** 31 - 1, 1, "too many tokens"), (2 ** 31 - 63, 1, "too many tokens"),
+    (2 ** 30, 64, "too many tokens"), (1, 2 ** 30 + 2, "GQA group")])
+def test_causal_attention_rejects_block_numbers_past_int32(tokens, kv_heads, message):
+    heads = (4 * kv_heads + 2 ** 31) % 2 ** 32 - 2 ** 31       # as int32 wraps it
+    rc, text = _call("pg_causal_attention", FAKE, MOST - 7, FAKE, MOST - 7, FAKE, MOST - 7, FAKE,
+                     MOST - 7, tokens, heads, kv_heads, 0.1, None)
+    assert rc != 0 and message in text
+
+
+@pytest.mark.parametrize("tokens,query_heads,kv_heads", [
+    (1, 2 ** 31 - 1, 2 ** 31 - 1), (2 ** 60, 32, 8), (1, 2 ** 24, 1)])
+def test_rope_rows_rejects_sizes_past_int32(tokens, query_heads, kv_heads):
+    rc, text = _call("pg_rope_rows", FAKE, MOST - 7, FAKE, FAKE, 128, FAKE, FAKE, tokens,
+                     query_heads, kv_heads, None)
+    assert rc == 1 and "too many tokens" in text
