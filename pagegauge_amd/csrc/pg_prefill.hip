@@ -35,6 +35,9 @@ constexpr int kTileKeys = 64;
 constexpr int kTileBytes = kTileKeys * kHeadDim * 2;     // 16 KiB
 constexpr float kRescaleLimit = 8.0f;                    // log2
 constexpr float kNegInf = -__builtin_huge_valf();
+// The running maximum before the first finite score.  Finite, so that a tile
+// of -inf scores adds probabilities of 0 and not exp2(-inf + inf).
+constexpr float kLowest = -__FLT_MAX__;
 
 struct AttentionArgs {
   const uint16_t* query;
@@ -152,7 +155,7 @@ __global__ __launch_bounds__(kWave * kWaves, 2) void causal_attention_kernel(Att
   for (int d = 0; d < 4; ++d)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[d][r] = 0.0f;
-  float m = kNegInf, l = 0.0f, l1 = 0.0f;
+  float m = kLowest, l = 0.0f, l1 = 0.0f;
 
   auto qk = [&](int buffer, v16f (&s)[2]) {
 #pragma unroll

@@ -49,6 +49,35 @@ def test_causal_attention_matches_float64(cuda, tokens, kv_heads, scale):
         assert ((got[:, h] - want).abs() <= bound).all(), (h, ((got[:, h] - want).abs() / bound).max())
 
 
+@pytest.mark.parametrize("tokens,kv_heads", [(200, 2), (4099, 8)])        # 4 and 8 waves
+def test_causal_attention_of_infinite_scores(cuda, tokens, kv_heads):
+    """Keys of -inf scores weigh nothing, whole tiles of them from the first
+    key on included; a row of nothing else, an infinite maximum and a NaN give
+    NaN rows, and every other row stays finite."""
+    from pagegauge_amd import decoder as dec
+
+    print(f"causal attention, infinite scores, tokens={tokens} kv_heads={kv_heads}", flush=True)
+    q, k, v = _prompt(tokens, kv_heads, 1.0, cuda)
+    q[..., 0] = q[..., 0].abs() + 0.5
+    k[..., 0] = 0.0
+    dead = list(range(0, 70)) + [100, 131]                  # past the first tile of 64
+    k[dead, :, 0] = float("-inf")
+    q[150], k[170, :, 0], q[:, 3, 0] = float("nan"), float("inf"), 0.25
+    got = dec._causal_attention(q, k, v)
+    rows = torch.arange(tokens, device=cuda)
+    hidden = rows[None, :] > rows[:, None]
+    nan = (rows < 70) | (rows == 150) | (rows >= 170)
+    for h in range(0, q.shape[1], 3):
+        scores = (q[:, h].double() @ k[:, h // 4].double().t()) * 128 ** -0.5
+        p = torch.softmax(scores.masked_fill(hidden, float("-inf")), dim=-1)
+        want = p @ v[:, h // 4].double()
+        assert torch.equal(want.isnan().any(-1), nan) and torch.equal(got[:, h].isnan().all(-1), nan)
+        # FP16 probabilities and output, as in the test above (scale 1)
+        bound = ((2.0 ** -11 + 2.0 ** -13) * (p @ v[:, h // 4].double().abs() + want.abs())
+                 + tokens * 2.0 ** -25 * v.double().abs().max())
+        assert ((got[:, h].double() - want).abs() <= bound)[~nan].all(), h
+
+
 def test_causal_attention_takes_other_layouts_through_torch(cuda):
     from pagegauge_amd import decoder as dec
 
