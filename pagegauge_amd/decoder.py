@@ -178,6 +178,8 @@ def qkv_rope_append(weight: torch.Tensor, x: torch.Tensor, *, norm_weight: torch
     ``projection`` followed by ``rope_append_page_gauge_dynamic`` /
     ``rope_append_fp16_dynamic``, except that the PageGauge page finalize is
     left to the decode (``finalize=`` of its run)."""
+    if norm_weight is None:
+        raise ValueError("norm weight must be FP16 [K]")
     _qkv_rope_append("pg_decoder_qkv_rope_append", weight, x, norm_weight, eps, query_heads,
                      kv_heads, cos, sin, positions, rotated_query, key_pages, value_pages,
                      key_center, value_center, pages_per_request, sink_pages, capacity_tokens)

@@ -65,6 +65,24 @@ def test_norm_rows_refuses_other_shapes(monkeypatch, weight, delta):
     assert len(launches) == 1
 
 
+def test_qkv_rope_append_needs_its_norm_weight(monkeypatch):
+    """Without one the projection would run on rows that nothing normalised."""
+    from pagegauge_amd import _capi, decoder as dec
+
+    launches = []
+    monkeypatch.setattr(_capi, "call", lambda *args: launches.append(args))
+    pages = torch.zeros(4, 16, 1, 128, dtype=H)
+    with pytest.raises(ValueError, match="norm weight"):
+        dec.qkv_rope_append(torch.zeros(768, 4096, dtype=H), torch.zeros(1, 4096, dtype=H),
+                            norm_weight=None, eps=1e-5, query_heads=4, kv_heads=1,
+                            cos=torch.zeros(64, 128, dtype=H), sin=torch.zeros(64, 128, dtype=H),
+                            positions=torch.zeros(1, dtype=torch.int32),
+                            rotated_query=torch.zeros(1, 4, 128, dtype=H), key_pages=pages,
+                            value_pages=pages, key_center=None, value_center=None,
+                            pages_per_request=4, sink_pages=0, capacity_tokens=64)
+    assert not launches
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("name", ["input_norm", "post_norm", "norm"])
 def test_one_element_norm_weights_broadcast(cuda, name):
