@@ -783,18 +783,18 @@ class PageGaugeDecoder:
         if self.fused and not ok:
             raise ValueError("fused projections need batch <= 4 and widths that are multiples "
                              "of 512 (4096 / 14336, or batch * width <= 32768)")
-        # the QKV projection carries the cache update (pg_decoder_qkv_rope_append;
-        # the PageGauge page finalize then runs in the decode's FP16 pass)
         append_ok = self.fused and cfg.hidden == 4096
-        self.fused_append = append_ok if fused_append is None else fused_append
-        if self.fused_append and not append_ok:
+        if fused_append and not append_ok:
             raise ValueError("the fused cache update needs fused projections and hidden 4096")
         # larger batches: the same steps through the matrix-core projections,
         # where the weights are laid out as they read them; otherwise (and with
         # ``fused=False``) torch operators
         self.batched = (fused is None and not ok and self._matrix_projections_take(weights,
                                                                                     batch_size))
-        self._append_in_projection = self.fused_append or (self.batched and fused_append is None)
+        # whether the QKV projection carries the cache update
+        # (pg_decoder_qkv_rope_append, pg_decoder_gemm_rope_append; the PageGauge
+        # page finalize then runs in the decode's FP16 pass)
+        self.fused_append = append_ok or self.batched if fused_append is None else fused_append
         self._projection_entry = "pg_decoder_gemm" if self.batched else "pg_decoder_gemv"
         self._append_entry = ("pg_decoder_gemm_rope_append" if self.batched
                               else "pg_decoder_qkv_rope_append")
@@ -970,8 +970,7 @@ class PageGaugeDecoder:
         c = self.cache
         value_center = c.value_center[layer]
         # with the fused cache update, the decode finalizes a completed page
-        finalize = ((self.device_position, c.pages_per_request) if self._append_in_projection
-                    else None)
+        finalize = (self.device_position, c.pages_per_request) if self.fused_append else None
         if self.tail_attention == "heterogeneous":
             return self.decode.run(self.rotated_query, (c.key_codes[layer], c.value_codes[layer]),
                                    c.key_scales[layer], c.value_scales[layer], c.exact_key[layer],
@@ -991,7 +990,7 @@ class PageGaugeDecoder:
         b = self.batch_size
         qw, kw = cfg.q_heads * DIM, cfg.kv_heads * DIM
         entry = self._projection_entry
-        if self._append_in_projection:
+        if self.fused_append:
             self._qkv_append(layer)
         else:
             x, norm = self._norm_input(w["input_norm"])

@@ -121,6 +121,8 @@ def test_batched_steps_match_torch_operator_steps(cuda, batch, backend):
     plain = dec.PageGaugeDecoder(weights, fast.cache.clone(), backend, fast.max_pages * 16,
                                  fast.rope_cos, fast.rope_sin, batch_size=batch, fused=False)
     assert fast.batched and not plain.batched and not fast.fused
+    # what the attribute says is what a step does: the QKV projection carries the update
+    assert fast.fused_append and not plain.fused_append
     token, kept = first, []
     for i in range(18):
         a, b = fast.step(token, 304 + i), plain.step(token, 304 + i)
