@@ -157,6 +157,11 @@ def _projection(entry: str, weight: torch.Tensor, x: torch.Tensor, out: torch.Te
     out_f32 = out.dtype == torch.float32
     if not out_f32 and out.dtype != torch.float16:
         raise ValueError("projection output must be FP16 or float32")
+    device = x.get_device()
+    if (device < 0 or weight.get_device() != device or out.get_device() != device
+            or (norm_weight is not None and norm_weight.get_device() != device)
+            or (residual is not None and residual.get_device() != device)):
+        raise ValueError("projection operands must be on one CUDA device")
     _capi.call(entry, weight.data_ptr(), n, k, x.data_ptr(), x.stride(0), batch,
                None if norm_weight is None else norm_weight.data_ptr(), float(eps), int(swiglu),
                None if residual is None else residual.data_ptr(),

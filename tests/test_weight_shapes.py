@@ -1,6 +1,6 @@
 """Weights whose shapes are not the configured ones stay off the kernels that
 take their sizes from the configuration: torch operators broadcast or refuse
-them as they always did, and no kernel reads past them."""
+them as they always did, and no kernel reads past them or off the device."""
 
 from __future__ import annotations
 
@@ -80,6 +80,20 @@ def test_qkv_rope_append_needs_its_norm_weight(monkeypatch):
                             rotated_query=torch.zeros(1, 4, 128, dtype=H), key_pages=pages,
                             value_pages=pages, key_center=None, value_center=None,
                             pages_per_request=4, sink_pages=0, capacity_tokens=64)
+    assert not launches
+
+
+@pytest.mark.parametrize("entry", ["pg_decoder_gemv", "pg_decoder_gemm"])
+def test_projections_refuse_host_operands(monkeypatch, entry):
+    """A weight left on the host raises, as it does in torch operators."""
+    from pagegauge_amd import _capi, decoder as dec
+
+    launches = []
+    monkeypatch.setattr(_capi, "call", lambda *args: launches.append(args))
+    monkeypatch.setattr(_capi, "current_stream", lambda: 0)
+    with pytest.raises(ValueError, match="one CUDA device"):
+        dec._projection(entry, torch.zeros(16, 512, dtype=H), torch.zeros(6, 512, dtype=H),
+                        torch.zeros(6, 16, dtype=H), None, 1e-5, False, None)
     assert not launches
 
 
