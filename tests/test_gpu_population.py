@@ -25,6 +25,8 @@ def _source(kind, tokens, heads, pad, device):
     elif kind == "outliers":
         x[..., ::32] *= 8
         x[16:32] = 0.0                                  # an all-zero page
+    elif kind == "nan":                                 # a finite scale: the products' path
+        x[3, :, 5], x[21, :, 9] = float("nan"), float("nan")
     elif kind == "not_finite":
         x[3, :, 5], x[20, :, 7], x[20, :, 9] = float("inf"), float("nan"), float("-inf")
     rows = torch.zeros(tokens, heads * 128 + pad, device=device, dtype=torch.float16)
@@ -33,7 +35,7 @@ def _source(kind, tokens, heads, pad, device):
     return out
 
 
-@pytest.mark.parametrize("kind", ["plain", "outliers", "tiny", "large", "not_finite"])
+@pytest.mark.parametrize("kind", ["plain", "outliers", "tiny", "large", "nan", "not_finite"])
 @pytest.mark.parametrize("pages,heads", [(3, 8), (5, 1), (33, 3)])
 def test_prefill_widths_agree(cuda, kind, pages, heads):
     from pagegauge_amd.update import prefill_page_gauge
@@ -54,7 +56,7 @@ def test_prefill_widths_agree(cuda, kind, pages, heads):
         assert torch.equal(_bits(wide), _bits(narrow))
 
 
-@pytest.mark.parametrize("kind", ["outliers", "tiny", "large", "not_finite"])
+@pytest.mark.parametrize("kind", ["outliers", "tiny", "large", "nan", "not_finite"])
 def test_half_even_widths_agree(cuda, kind):
     from pagegauge_amd.update import quantize_page_gauge
 

@@ -63,6 +63,25 @@ def test_swiglu_rows(cuda, rows, width):
     assert (got != want).float().mean() < 1e-2
 
 
+def test_rows_of_extreme_values(cuda):
+    """Infinities, NaN and the largest values, as torch operators take them."""
+    from pagegauge_amd import decoder as dec
+
+    inf, nan = float("inf"), float("nan")
+    extreme = torch.tensor([inf, -inf, nan, 65504.0, -65504.0, 6e-8, -0.0, 1.0], device=cuda).half()
+    gate_up = torch.cat((extreme.repeat_interleave(8), extreme.repeat(8))).view(1, 128)
+    gate, up = gate_up.split(64, dim=-1)
+    assert torch.equal(dec._swiglu_rows(gate_up).nan_to_num(5.0, 7.0, -7.0),
+                       (F.silu(gate) * up).nan_to_num(5.0, 7.0, -7.0))
+    x = torch.stack([_rand(cuda, 64) for _ in range(8)])
+    x[:, 3] = extreme
+    want = dec.rms_norm(x, torch.ones(64, device=cuda).half(), 1e-5)
+    got = dec._norm_rows(x, torch.ones(64, device=cuda).half(), 1e-5, None)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    got, want = (t.float().nan_to_num(0.0) for t in (got, want))
+    assert ((got - want).abs() <= want.abs() * 2.0 ** -9 + 2.0 ** -23).all()
+
+
 def test_prefill_with_kernels_matches_torch_operators(cuda, monkeypatch):
     from pagegauge_amd import decoder as dec
 
