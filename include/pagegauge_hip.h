@@ -324,9 +324,9 @@ int64_t pg_decode_workspace_bytes(int32_t batch_size, int32_t num_qo_heads,
 
 /* Split selection: the pages per work item that pg_decode_plan's balanced
  * planner (split_pages <= 0) chooses on num_cus CUs for batch_size requests
- * sharing total_pages pages evenly, with no tail segment.  bytes_per_page is
- * the per-(page, kv head) K+V traffic: 4096 plans INT8 pages, 8192 FP16
- * pages.  Returns 0 (message in pg_last_error) for invalid arguments or a
+ * sharing total_pages pages evenly, with no tail segment, in a workspace that
+ * holds its plan.  bytes_per_page is the per-(page, kv head) K+V traffic: 4096
+ * plans INT8 pages, 8192 FP16 pages.  Returns 0 (message in pg_last_error) for invalid arguments or a
  * batch the planner cannot cut.  Replaces FlashInfer's automatic split
  * (fixed_split_size=None) and the capacity bound (2*num_SMs)//Hkv of
  * diagnostics/benchmark_sustained_dynamic_graphs.py:1497-1534. */
@@ -340,8 +340,14 @@ int32_t pg_select_split_pages(int64_t total_pages, int32_t batch_size, int32_t n
  * items (the item count of FlashInfer's fixed_split_size, balanced sizes);
  * the tail likewise with tail_split_pages, default ceil(split_pages/2) for
  * INT8 (an FP16 page streams twice the bytes);
- * split_pages <= 0 balances the batch over num_cus workgroups (every item at
- * most 64 pages, FP16 pages weighted twice INT8 pages).
+ * split_pages <= 0 balances the batch (every item at most 64 pages, FP16
+ * pages weighted twice INT8 pages): over num_cus workgroups, fewer items where
+ * two workgroups share each, and up to 3/2 * num_cus items where one round
+ * would stay uneven.  Where workspace_bytes does not hold that last kind of
+ * plan, the batch is planned again with the fewest items; so the items, and
+ * with them the last bits of the outputs, depend on the workspace's size up to
+ * plan->workspace_bytes of the fuller plan (pg_decode_plan_host's), and on
+ * nothing past it.
  * exact_tail_pages_hint (heterogeneous plans only, else 0): the number of
  * trailing pages of each request's unified table expected to be FP16 exact
  * pages at run time; they are planned like a tail segment (own items,
@@ -360,7 +366,8 @@ int32_t pg_decode_plan(const int32_t* host_indptr, const int32_t* host_last_page
                        int64_t workspace_bytes, pg_decode_plan_t* plan, void* stream);
 
 /* The host half of pg_decode_plan (same arguments, same validation and
- * errors) without a device: fills *plan and, if items_out != NULL, the work
+ * errors, for a workspace of any size: the plan of one that holds
+ * plan->workspace_bytes) without a device: fills *plan and, if items_out != NULL, the work
  * list as 12 int32 per item (items_capacity counts items, so items_out holds
  * 12 * items_capacity int32) {request, kind (PG_KV_*), segment (0 primary,
  * 1 tail), page_begin, page_end (positions in indices/tail_indices), last

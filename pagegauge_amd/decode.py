@@ -195,9 +195,10 @@ def plan_work_items(indptr, last_page_len, tail_indptr=None, tail_last_page_len=
     """Run the decode scheduler on the host only (no device, no workspace).
 
     Returns ``(plan, items, item_ptr)``: the ``DecodePlan`` that
-    ``pg_decode_plan`` would produce, the work list as an int32 tensor
-    [num_items, 12] with columns ``WORK_ITEM_FIELDS``, and [B+1] per-request
-    item offsets.  Same validation and error messages as ``plan``.
+    ``pg_decode_plan`` produces in a workspace of at least its
+    ``workspace_bytes`` (a smaller one may get fewer items), the work list as
+    an int32 tensor [num_items, 12] with columns ``WORK_ITEM_FIELDS``, and
+    [B+1] per-request item offsets.  Same validation and error messages as ``plan``.
     """
     lib = _capi.library()
     host_indptr, host_last = _host_tables(indptr, last_page_len)

@@ -100,3 +100,71 @@ def test_both_plans_of_a_batch_match_attention(cuda, pages):
         ref = (p[:, :, None] * v).sum(0)
         for _, out in outs:
             assert max_abs(out[b], ref.cpu()) <= 2e-3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,old,exact", [
+    ("heterogeneous", [70, 70, 90, 100, 127, 60, 50], 4), ("heterogeneous", MEDIUM, 3),
+    ("segmented", [120, 120, 60, 40], 16), ("segmented", [50, 64, 30, 20, 44], 8)])
+def test_both_plans_of_a_compressed_batch_match_attention(cuda, kind, old, exact):
+    """The same over an INT8 history and exact pages, as two segments and as
+    one table: the fuller plan and the fewest items (in a workspace of just
+    their size) against attention in float64 over the dequantised pages (2e-3
+    as above)."""
+    import re
+
+    from pagegauge_amd import decode
+
+    g = torch.Generator(device=cuda).manual_seed(6)
+    batch, total, tails = len(old), sum(old), exact * len(old)
+
+    def normal(*shape):
+        return torch.randn(*shape, device=cuda, generator=g)
+
+    codes = [normal(total, 16, 8, 128).mul(40).round().clamp(-127, 127).to(torch.int8) for _ in range(2)]
+    scales = [(normal(total, 8).abs() * 0.01 + 0.02).half() for _ in range(2)]
+    pages = [normal(tails, 16, 8, 128).half() for _ in range(2)]
+    query, center = normal(batch, 32, 128).half(), (normal(batch, 8, 128) * 0.1).half()
+    old_ids = torch.randperm(total, device=cuda, generator=g).int()
+    exact_ids = torch.randperm(tails, device=cuda, generator=g).int()
+    last = torch.tensor([16 - b % 5 for b in range(batch)], dtype=torch.int32, device=cuda)
+    ends = np.concatenate([[0], np.cumsum(old)]).astype(np.int32)
+    old_ptr, exact_ptr = torch.tensor(ends), torch.arange(0, tails + 1, exact, dtype=torch.int32)
+    full = torch.full((batch,), 16, dtype=torch.int32, device=cuda)
+    unified = torch.cat([t for b in range(batch)
+                         for t in (old_ids[ends[b]:ends[b + 1]], exact_ids[b * exact:(b + 1) * exact])])
+    old_kv_len = torch.tensor(old, dtype=torch.int32, device=cuda) * 16
+
+    def attend(size):
+        ws = torch.empty(size, device=cuda, dtype=torch.uint8)
+        out = dict(value_center=center, return_lse=True)
+        if kind == "segmented":
+            d = decode.PageGaugeSegmentedDecode(ws)
+            d.plan(old_ptr, old_ids, full, exact_ptr, exact_ids, last, num_cus=CUS)
+            result = d.run(query, codes, *scales, pages, **out)
+        else:
+            d = decode.HeterogeneousDecodeWrapper(ws)
+            d.plan(old_ptr + exact_ptr, unified, last, num_cus=CUS, exact_tail_pages_hint=exact)
+            result = d.run(query, codes, *scales, *pages, old_kv_len, **out)
+        return d.num_work_items, [t.clone() for t in result]
+
+    with pytest.raises(RuntimeError, match="workspace too small") as refused:
+        attend(512)
+    small = int(re.search(r"need (\d+) bytes", str(refused.value)).group(1))
+    (most, fuller), (least, fewest) = attend(1 << 22), attend(small)
+    assert least < most <= CUS * 3 // 2
+    for b in range(batch):
+        rows = old_ids[ends[b]:ends[b + 1]].long()
+        tail = exact_ids[b * exact:(b + 1) * exact].long()
+        tokens = (exact - 1) * 16 + int(last[b])
+        k, v = (torch.cat(((c[rows].double() * s[rows].double()[:, None, :, None]).reshape(-1, 8, 128),
+                           p[tail].double().reshape(-1, 8, 128)[:tokens])).repeat_interleave(4, dim=1)
+                for c, s, p in zip(codes, scales, pages))
+        scores = (k * query[b].double()).sum(-1) * 128 ** -0.5
+        p = torch.softmax(scores, dim=0)
+        want = (p[:, :, None] * v).sum(0) + center[b].double().repeat_interleave(4, dim=0)
+        lse = torch.logsumexp(scores, dim=0) / np.log(2.0)
+        for out, got_lse in (fuller, fewest):
+            # beyond the output's own FP16 rounding
+            excess = (out[b].double() - want).abs() - want.abs() * 2.0 ** -11
+            assert float(excess.max()) <= 2e-3 and max_abs(got_lse[b], lse.cpu()) <= 2e-3
