@@ -75,8 +75,9 @@ struct AttentionArgs {
 // The running maximum is raised only when a score exceeds it by more than
 // 2^8 (probabilities then reach 256, which FP16 holds at the same relative
 // precision): most tiles skip the rescale of the accumulators.  A lane adds its
-// probabilities in float32, in two sums: half the chain, half the terms in each
-// (16384 tokens 2036 us with one, 2032 with two; 1000 tokens 22.8 both).
+// probabilities in float32, in two sums: half the chain (16384 tokens 2047 us
+// with one, 2044 with two; no difference at 1000 tokens, nor in the error
+// against 64 bits at any length).
 //
 // Blocks are dispatched longest first, and KV heads vary fastest, so that with
 // 8 heads each XCD works on one head's keys and values.

@@ -13,7 +13,13 @@ completes and finalizes leave the ring from position 640 on.
   INT8 pool or its exact slot; not from the decoder's tables): within 2e-3
   beyond half an FP16 ulp of the dense value.
 * At positions across those transitions, the logits against the same step
-  with dense attention, within max(2e-3, the decoder's FP16 rounding floor).
+  with dense attention, within what FP16 rounding of the attention's output
+  makes of them: a step's floor is the distance between its logits with the
+  dense attention rounded to FP16 and unrounded.  Either side of the comparison
+  rounds its attention, so each may lie a floor from the unrounded step and the
+  two up to twice that apart (or 2e-3).  A single position's floor is one draw
+  of rounding noise, as is its distance; the largest of the nine positions
+  stands for all.
 * The suffix slots hold the prefill's rows after 140 steps (no ring write
   lands on them), and graph replay equals eager steps bit for bit.
 """
@@ -98,9 +104,10 @@ def test_static_suffix_decode_against_dense_attention(setup):
         walker.step(tokens[i:i + 1], position)
         assert walker.kernel_error <= 2e-3, position          # K1 against dense, every step
     print(f"worst attention excess over {STEPS} steps: {walker.kernel_error:.3g}", flush=True)
+    worst = max(floor for _, _, floor in rows)
     for position, distance, floor in rows:
         assert floor <= FLOOR_BOUND, position
-        assert distance <= max(2e-3, floor), position
+        assert distance <= max(2e-3, 2 * worst), position
     # the suffix slots were never written by the ring
     assert torch.equal(walker.cache.exact_key[:, suffix_slots], suffix_rows)
     # the tail has moved past the suffix: pages 24..27 and the decode's first
