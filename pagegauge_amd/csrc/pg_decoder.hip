@@ -484,9 +484,9 @@ __global__ __launch_bounds__(kGemvThreads) void decoder_gemv_generic_kernel(Gemv
 // with SwiGLU; dims d..d+7 and d+64..d+71 of one head for the append), each of
 // its 8 waves an eighth of the input width; the waves' 16 x 16 sums meet in
 // LDS (two buffers, one barrier per tile).  One workgroup per CU walks the
-// tiles, and a wave keeps two tiles of its slice (32 KiB) in flight, in blocks
-// of 4 KiB that are refilled one by one, so that the stream does not stop
-// at a tile's reduction.
+// tiles, and a wave keeps blocks of 4 KiB of weights in flight that are refilled
+// one by one, so that the stream does not stop at a tile's reduction: two tiles
+// of its slice (32 KiB) with a resident input, two blocks with a streamed one.
 //
 // The operands want 16 rows x 64 bytes per load: half cache lines.  Here a load
 // takes 8 rows x 128 bytes instead, of weights and of inputs, its lanes r < 8
@@ -812,14 +812,19 @@ int32_t launch_matrix(const GemvArgs& a, int batch, hipStream_t s, const char* w
   return check_launch(what);
 }
 
-// Whether a batch of 1 to 4 rows runs on the matrix cores: at the widths with
-// kernels of their own, from 3 rows on, and with 2 rows except behind a norm
-// without SwiGLU (QKV, head), where the v_dot2 kernel is the faster one (figures
-// above).  At other widths the staged kernel stays ahead up to 4 rows (us for 2
-// / 4 rows, staged against streamed: 5120 x 5120 12.2 / 14.4 against 15.7 /
-// 16.8, 2048 x 5632 8.1 / 10.4 against 9.3 / 10.0).  The rule looks at nothing
-// but the projection, so that the QKV projection with and without the cache
-// update gives the same bits.
+// Whether a batch of 1 to 4 rows runs on the matrix cores.  4096 and 14336 are
+// the widths whose v_dot2 kernels keep every row's input in registers (the
+// others stage it in LDS): from 3 rows on the matrix cores are faster there,
+// and with 2 rows except behind a norm without SwiGLU (QKV, head; figures
+// above), so those kernels are not built for more rows.  At the other widths no
+// threshold in the width tells the faster one (us for 2 / 3 / 4 rows, staged
+// against streamed: 1024 x 1024 3.5 / 4.2 / 4.8 and 3.3 / 3.4 / 3.5, 2048 x 5632
+// 8.2 / 9.2 / 10.2 and 9.0 / 9.3 / 9.6, 5120 x 5120 13.0 / 14.1 / 14.9 and 16.1 /
+// 16.7 / 16.5, 4096 x 8192 15.6 / 16.8 / 17.9 and 14.3 / 14.5 / 14.9; 2 rows of
+// 5120 x 13824 34.4 and 37.6, 4096 x 16384 33.4 and 35.3, 1024 x 16384 13.6 and
+// 19.5): they stay with the staged kernel, within its LDS.  The rule looks at
+// nothing but the projection, so that the QKV projection with and without the
+// cache update gives the same bits.
 bool matrix_batch(const GemvArgs& a, int batch) {
   const bool own_width = a.k == kResidentWidth || (a.k == 14336 && !a.swiglu && !a.norm_weight);
   if (!own_width || batch < 2) return false;

@@ -248,6 +248,9 @@ int32_t build_plan(const int32_t* host_indptr, const int32_t* host_last_page_len
       // 118 us; B95 x 1.5K FP16, 256 items: 117 us, 380: 110 us.  An even
       // round is the better one (B8 ragged, 256 items: 64 us, 384: 67 us).
       // Segmented plans whose uncut items pass one round keep those items.
+      // Against the fewest items over 70 drawn uneven batches (8 to 245 requests,
+      // 300 to 55000 tokens, all three forms): 0.97 to 1.43 times as fast, 1.07
+      // in the middle, three of them slower by more than 1 %.
       std::vector<int> cut(segments.size(), 0);
       count_for(hi, &cut);
       double heaviest = 0.0;

@@ -422,7 +422,8 @@ typedef uint32_t v2u __attribute__((ext_vector_type(2)));
 // error of 2^-24, that is within 2^-23 ulp of the true quotient before its
 // rounding.  A quotient of a 24-bit by an 11-bit number is never a midpoint
 // of two floats and lies at least 2^-12 ulp from one, so q is correctly
-// rounded.  An infinite scale (infinite or NaN input) takes the division.
+// rounded.  An infinite scale (of an infinite input) takes the division; a NaN,
+// which the maximum passes over, is a NaN quotient either way and gives 0.
 __device__ __forceinline__ void quantize_rows(const v4u (&rows)[4], v4u center, int64_t row_stride,
                                               int8_t* codes, uint16_t* scale_out, uint16_t* ring,
                                               int lane, bool half_even) {

@@ -443,10 +443,10 @@ def _prefill_layers(weights: DecoderWeights, hidden: torch.Tensor, cos: torch.Te
 
 def _head_rows(weights: DecoderWeights, last: torch.Tensor) -> torch.Tensor:
     """Final norm and LM head of one row: float32 logits [1, vocab], one launch
-    of the decode step's projection where its width allows (multiples of 512
-    up to 32768: 43 against 91 us as norm, GEMM and cast at 4096 x 32768)."""
+    of the decode step's projection where its width allows (multiples of 512:
+    43 against 91 us as norm, GEMM and cast at 4096 x 32768)."""
     cfg = weights.config
-    if cfg.hidden % 512 or cfg.hidden > 32768 or not all(
+    if cfg.hidden % 512 or not all(
             w.is_contiguous() and w.data_ptr() % 16 == 0 for w in (weights.lm_head, weights.norm)):
         return F.linear(rms_norm(last, weights.norm, cfg.rms_eps), weights.lm_head).float()
     logits = torch.empty(1, weights.lm_head.shape[0], device=last.device, dtype=torch.float32)
