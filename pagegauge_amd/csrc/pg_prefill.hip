@@ -66,9 +66,9 @@ struct AttentionArgs {
 // source address) so that neither the K reads (8 rows per access) nor the
 // transposing V reads (4 rows x 32 bytes) meet in a bank.  The scores of tile
 // j + 1 are computed beside the softmax of tile j: the two halves of the work
-// use the matrix cores and the VALU (exp2 at a quarter rate) for about the
-// same time, which is what bounds the kernel, with the LDS reads (32 KiB per
-// wave and tile) close behind.
+// use the matrix cores and the VALU for about the same time (58 and 54 % of the
+// cycles at 16384 tokens), which is what bounds the kernel; the LDS reads (32 KiB
+// per wave and tile) take half of either.
 //
 // The running maximum is raised only when a score exceeds it by more than
 // 2^8 (probabilities then reach 256, which FP16 holds at the same relative
